@@ -29,8 +29,8 @@
 // row-major tile with ds_read_b64_tr_b16.  Eight-wave workgroups share each
 // streamed tile between twice as many rows, halving the L2 -> LDS bytes per
 // FLOP; attn_waves (attn_fwd.hip) picks the shape.
-// All GEMMs run on v_mfma_f32_32x32x16_bf16 (bf16 storage) or
-// v_mfma_f32_32x32x2_f32 (f32 storage) with f32 accumulation.
+// All GEMMs run on v_mfma_f32_32x32x16_bf16 with f32 accumulation.  f32
+// storage has its own dK/dV and dQ (attn_f32.hip) and shares the delta pass.
 #include <math.h>
 
 #include "fa_device.hpp"
@@ -882,167 +882,6 @@ hipError_t launch_reduce(const AttnBwdParams &p, int D, int z0, int nz, hipStrea
     return hipGetLastError();
 }
 
-// ---------------------------------------------------------------------------
-// f32 backward (FA_DTYPE_F32): exact f32 MFMA, one wave per 32 keys (dK/dV)
-// or 32 queries (dQ), 32-row blocks.  Parity path for the reference's f32 run.
-// ---------------------------------------------------------------------------
-template <int D>
-__global__ __launch_bounds__(64) void attn_bwd_dkdv_f32_kernel(AttnBwdParams p) {
-    __shared__ float Qs[32][D + 1];
-    __shared__ float Os[32][D + 1];  // dO block
-    __shared__ float Ls[32], Ds[32];
-    const int lane = threadIdx.x, n = lane & 31, g = lane >> 5;
-    const int S = p.S, H = p.H;
-    const int nk = (S + 31) / 32;
-    const int kt = blockIdx.x % nk, bh = blockIdx.x / nk;
-    const int h = bh % H, b = bh / H;
-    const float *qbase = static_cast<const float *>(p.q) + b * p.q_sb + h * p.q_sh;
-    const float *kbase = static_cast<const float *>(p.k) + b * p.k_sb + h * p.k_sh;
-    const float *vbase = static_cast<const float *>(p.v) + b * p.v_sb + h * p.v_sh;
-    const float *dobase = static_cast<const float *>(p.dout) + b * p.do_sb + h * p.do_sh;
-    const float *lse = p.lse + ((int64_t)b * H + h) * S;
-    const float *delta = p.delta + ((int64_t)b * H + h) * S;
-    const int kj = kt * 32 + n;
-    const bool kept = kj < S && (!p.keep || p.keep[(int64_t)b * S + kj]);
-    float kf[D / 2], vf[D / 2];
-#pragma unroll
-    for (int kd = 0; kd < D / 2; ++kd) {
-        kf[kd] = kj < S ? kbase[kj * p.k_ss + 2 * kd + g] : 0.f;
-        vf[kd] = kj < S ? vbase[kj * p.v_ss + 2 * kd + g] : 0.f;
-    }
-    f32x16 dk[D / 32], dv[D / 32];
-#pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) dk[dt][r] = dv[dt][r] = 0.f;
-    const float c = p.scale_log2;
-    for (int q0 = 0; q0 < S; q0 += 32) {
-        __syncthreads();
-        for (int e = lane; e < 32 * D; e += 64) {
-            const int row = e / D, d = e % D, qi = q0 + row;
-            Qs[row][d] = qi < S ? qbase[qi * p.q_ss + d] : 0.f;
-            Os[row][d] = qi < S ? dobase[qi * p.do_ss + d] : 0.f;
-        }
-        if (lane < 32) {
-            const int qi = q0 + lane;
-            const float l = qi < S ? lse[qi] : INFINITY;
-            Ls[lane] = l == -INFINITY ? INFINITY : l * kLog2e;
-            Ds[lane] = qi < S ? delta[qi] : 0.f;
-        }
-        __syncthreads();
-        f32x16 s, dp;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
-#pragma unroll
-        for (int kd = 0; kd < D / 2; ++kd) {
-            s = mfma_32x32x2_f32(Qs[n][2 * kd + g], kf[kd], s);
-            dp = mfma_32x32x2_f32(Os[n][2 * kd + g], vf[kd], dp);
-        }
-        f32x16 pm, dsm;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int qi = acc_row(r, lane);
-            const float pv = kept ? exp2f(s[r] * c - Ls[qi]) : 0.f;
-            pm[r] = pv;
-            dsm[r] = pv * (dp[r] - Ds[qi]);
-        }
-#pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-            for (int t = 0; t < 16; ++t) {
-                const int qi = acc_row(t, lane);
-                dv[dt] = mfma_32x32x2_f32(pm[t], Os[qi][dt * 32 + n], dv[dt]);
-                dk[dt] = mfma_32x32x2_f32(dsm[t], Qs[qi][dt * 32 + n], dk[dt]);
-            }
-    }
-    float *dkb = static_cast<float *>(p.dk) + b * p.dk_sb + h * p.dk_sh;
-    float *dvb = static_cast<float *>(p.dv) + b * p.dv_sb + h * p.dv_sh;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int key = kt * 32 + acc_row(r, lane);
-        if (key < S)
-#pragma unroll
-            for (int dt = 0; dt < D / 32; ++dt) {
-                dkb[key * p.dk_ss + dt * 32 + n] = dk[dt][r] * p.scale;
-                dvb[key * p.dv_ss + dt * 32 + n] = dv[dt][r];
-            }
-    }
-}
-
-template <int D>
-__global__ __launch_bounds__(64) void attn_bwd_dq_f32_kernel(AttnBwdParams p) {
-    __shared__ float Ks[32][D + 1];
-    __shared__ float Vs[32][D + 1];
-    const int lane = threadIdx.x, n = lane & 31, g = lane >> 5;
-    const int S = p.S, H = p.H;
-    const int nq = (S + 31) / 32;
-    const int qt = blockIdx.x % nq, bh = blockIdx.x / nq;
-    const int h = bh % H, b = bh / H;
-    const float *qbase = static_cast<const float *>(p.q) + b * p.q_sb + h * p.q_sh;
-    const float *kbase = static_cast<const float *>(p.k) + b * p.k_sb + h * p.k_sh;
-    const float *vbase = static_cast<const float *>(p.v) + b * p.v_sb + h * p.v_sh;
-    const float *dobase = static_cast<const float *>(p.dout) + b * p.do_sb + h * p.do_sh;
-    const uint8_t *keep = p.keep ? p.keep + (int64_t)b * S : nullptr;
-    const int qi = qt * 32 + n;
-    float qf[D / 2], of[D / 2];
-#pragma unroll
-    for (int kd = 0; kd < D / 2; ++kd) {
-        qf[kd] = qi < S ? qbase[qi * p.q_ss + 2 * kd + g] : 0.f;
-        of[kd] = qi < S ? dobase[qi * p.do_ss + 2 * kd + g] : 0.f;
-    }
-    float lse2 = INFINITY, dlt = 0.f;
-    if (qi < S) {
-        const float l = p.lse[((int64_t)b * H + h) * S + qi];
-        lse2 = l == -INFINITY ? INFINITY : l * kLog2e;
-        dlt = p.delta[((int64_t)b * H + h) * S + qi];
-    }
-    f32x16 dq[D / 32];
-#pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) dq[dt][r] = 0.f;
-    const float c = p.scale_log2;
-    for (int k0 = 0; k0 < S; k0 += 32) {
-        __syncthreads();
-        for (int e = lane; e < 32 * D; e += 64) {
-            const int row = e / D, d = e % D, key = k0 + row;
-            Ks[row][d] = key < S ? kbase[key * p.k_ss + d] : 0.f;
-            Vs[row][d] = key < S ? vbase[key * p.v_ss + d] : 0.f;
-        }
-        __syncthreads();
-        bool kept = false;
-        if (lane < 32) kept = k0 + lane < S && (!keep || keep[k0 + lane]);
-        const uint64_t km = __ballot(kept);
-        f32x16 s, dp;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
-#pragma unroll
-        for (int kd = 0; kd < D / 2; ++kd) {
-            s = mfma_32x32x2_f32(Ks[n][2 * kd + g], qf[kd], s);
-            dp = mfma_32x32x2_f32(Vs[n][2 * kd + g], of[kd], dp);
-        }
-        f32x16 dsm;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int kk = acc_row(r, lane);
-            const float pv = ((km >> kk) & 1) ? exp2f(s[r] * c - lse2) : 0.f;
-            dsm[r] = pv * (dp[r] - dlt);
-        }
-#pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-            for (int t = 0; t < 16; ++t)
-                dq[dt] = mfma_32x32x2_f32(Ks[acc_row(t, lane)][dt * 32 + n], dsm[t], dq[dt]);
-    }
-    if (qi < S) {
-        float *row = static_cast<float *>(p.dq) + b * p.dq_sb + h * p.dq_sh + qi * p.dq_ss;
-#pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) row[dt * 32 + acc_row(r, lane)] = dq[dt][r] * p.scale;
-    }
-}
-
 template <typename T, int D>
 hipError_t launch_delta(const AttnBwdParams &p, hipStream_t s) {
     constexpr int LPR = D * sizeof(T) / 16;
@@ -1158,28 +997,8 @@ hipError_t launch_attn_bwd_bf16(const AttnBwdParams &p, int D, int phase, hipStr
     return e;
 }
 
-hipError_t launch_attn_bwd_f32(const AttnBwdParams &p, int D, int phase, hipStream_t s) {
-    hipError_t e = hipSuccess;
-    if (phase == 0 || phase == 1) {
-        e = D == 128 ? launch_delta<float, 128>(p, s) : launch_delta<float, 64>(p, s);
-        if (e != hipSuccess) return e;
-    }
-    const dim3 grid(p.B * p.H * ((p.S + 31) / 32)), block(64);
-    if (phase == 0 || phase == 2) {
-        if (D == 128)
-            hipLaunchKernelGGL(attn_bwd_dkdv_f32_kernel<128>, grid, block, 0, s, p);
-        else
-            hipLaunchKernelGGL(attn_bwd_dkdv_f32_kernel<64>, grid, block, 0, s, p);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-    }
-    if (phase == 0 || phase == 3) {
-        if (D == 128)
-            hipLaunchKernelGGL(attn_bwd_dq_f32_kernel<128>, grid, block, 0, s, p);
-        else
-            hipLaunchKernelGGL(attn_bwd_dq_f32_kernel<64>, grid, block, 0, s, p);
-        e = hipGetLastError();
-    }
-    return e;
+hipError_t launch_attn_bwd_delta_f32(const AttnBwdParams &p, int D, hipStream_t s) {
+    return D == 128 ? launch_delta<float, 128>(p, s) : launch_delta<float, 64>(p, s);
 }
 
 hipError_t prepare_bwd_kernels() { return hipSuccess; }  // static LDS only

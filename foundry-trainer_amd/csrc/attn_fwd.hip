@@ -485,104 +485,6 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(AttnFwdParams p) 
     if (c == 0) p.lse[row] = lse;
 }
 
-// ---------------------------------------------------------------------------
-// f32 forward (FA_DTYPE_F32): exact f32 products on v_mfma_f32_32x32x2_f32,
-// one wave per 32 queries, 32-key blocks.  This is the parity path for the
-// reference's f32 CPU run; P stays f32 as in lib.rs:147 for f32 inputs.
-// ---------------------------------------------------------------------------
-constexpr int kF32BN = 32;
-
-template <int D>
-__global__ __launch_bounds__(64) void attn_fwd_f32_kernel(AttnFwdParams p) {
-    __shared__ float Ks[kF32BN][D + 1];
-    __shared__ float Vs[kF32BN][D];
-    const int lane = threadIdx.x, n = lane & 31, g = lane >> 5;
-    const int S = p.S, H = p.H;
-    const int nq = (S + 31) / 32;
-    const int work = blockIdx.x;
-    const int qt = work % nq, bh = work / nq;
-    const int h = bh % H, b = bh / H;
-    const float *qbase = static_cast<const float *>(p.q) + b * p.q_sb + h * p.q_sh;
-    const float *kbase = static_cast<const float *>(p.k) + b * p.k_sb + h * p.k_sh;
-    const float *vbase = static_cast<const float *>(p.v) + b * p.v_sb + h * p.v_sh;
-    const uint8_t *keep = p.keep ? p.keep + (int64_t)b * S : nullptr;
-    const int qi = qt * 32 + n;
-
-    float qf[D / 2];
-#pragma unroll
-    for (int kd = 0; kd < D / 2; ++kd) qf[kd] = qi < S ? qbase[qi * p.q_ss + 2 * kd + g] : 0.f;
-    f32x16 o[D / 32];
-#pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
-    float m_run = -INFINITY, l_run = 0.f;
-    const float c = p.scale_log2;
-
-    for (int kb = 0; kb * kF32BN < S; ++kb) {
-        __syncthreads();
-        for (int e = lane; e < kF32BN * D; e += 64) {
-            const int row = e / D, d = e % D, key = kb * kF32BN + row;
-            Ks[row][d] = key < S ? kbase[key * p.k_ss + d] : 0.f;
-            Vs[row][d] = key < S ? vbase[key * p.v_ss + d] : 0.f;
-        }
-        __syncthreads();
-        bool kept = false;
-        if (lane < kF32BN) {
-            const int key = kb * kF32BN + lane;
-            kept = key < S && (!keep || keep[key]);
-        }
-        const uint64_t km = __ballot(kept);
-
-        f32x16 s;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = 0.f;
-#pragma unroll
-        for (int kd = 0; kd < D / 2; ++kd) s = mfma_32x32x2_f32(Ks[n][2 * kd + g], qf[kd], s);
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-            if (!((km >> acc_row(r, lane)) & 1)) s[r] = -INFINITY;
-
-        float mx = s[0];
-#pragma unroll
-        for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
-        mx = fmaxf(mx, xor32(mx));
-        const float m_new = fmaxf(m_run, mx);
-        const float m_sc = m_new == -INFINITY ? 0.f : m_new * c;
-        const float alpha = exp2f(m_run * c - m_sc);
-        m_run = m_new;
-        float psum = 0.f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            s[r] = exp2f(s[r] * c - m_sc);
-            psum += s[r];
-        }
-        l_run = l_run * alpha + psum;
-#pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const int key = acc_row(j, lane);  // key of element j in this lane half
-                o[dt] = mfma_32x32x2_f32(Vs[key][dt * 32 + n], s[j], o[dt]);
-            }
-        }
-    }
-    const float l_tot = l_run + xor32(l_run);
-    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    if (qi < S) {
-        float *orow = static_cast<float *>(p.o) + b * p.o_sb + h * p.o_sh + qi * p.o_ss;
-#pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) orow[dt * 32 + acc_row(r, lane)] = o[dt][r] * inv;
-        if (g == 0)
-            p.lse[((int64_t)b * H + h) * S + qi] =
-                l_tot > 0.f ? m_run * p.scale + logf(l_tot) : -INFINITY;
-    }
-}
-
 }  // namespace
 
 // Workgroup shape, shared by the forward and backward bf16 kernels.  An
@@ -685,16 +587,6 @@ hipError_t launch_attn_fwd_bf16(const AttnFwdParams &p, int D, hipStream_t s) {
         else
             hipLaunchKernelGGL((attn_fwd_bf16_kernel<64, 4, false, false>), grid, block, 0, s, p);
     }
-    return hipGetLastError();
-}
-
-hipError_t launch_attn_fwd_f32(const AttnFwdParams &p, int D, hipStream_t s) {
-    const int nq = (p.S + 31) / 32;
-    const dim3 grid(p.B * p.H * nq), block(64);
-    if (D == 128)
-        hipLaunchKernelGGL(attn_fwd_f32_kernel<128>, grid, block, 0, s, p);
-    else
-        hipLaunchKernelGGL(attn_fwd_f32_kernel<64>, grid, block, 0, s, p);
     return hipGetLastError();
 }
 

@@ -188,10 +188,11 @@ size_t bwd_min_workspace(int32_t dtype, int32_t B, int32_t S, int32_t H, int32_t
            3 * round256(fa::attn_split_elems(B, H, S, D, split) * sizeof(float));
 }
 
-// dS after that, for the backward whose dQ reads the dK/dV kernel's dS
-// (bf16, unsplit, 8-wave grids): per (b, h) S rounded up to 32 keys x ds_ld
-// queries bf16 (S rounded up to 256), in 1 KiB blocks of 32 keys x 16
-// queries.  0 where that path does not apply: f32, split calls, 4-wave grids
+// dS after that, for the backward whose dQ reads the dK/dV kernel's dS.
+// f32: per (b, h) S x S f32, both rounded up to 32, in 4 KiB blocks of 32 keys
+// x 32 queries.  bf16, unsplit 8-wave grids: per (b, h) S rounded up to 32
+// keys x ds_ld queries bf16 (S rounded up to 256), in 1 KiB blocks of 32 keys
+// x 16 queries.  0 where that path does not apply: split calls, 4-wave grids
 // (there the 4-wave dK/dV kernel's stores cost what dQ saves: c3 431 against
 // 450 us), or a head's blocks spanning 4 GiB (the kernels' buffer offsets
 // are 32-bit).
@@ -199,6 +200,12 @@ size_t bwd_min_workspace(int32_t dtype, int32_t B, int32_t S, int32_t H, int32_t
 // rather than ask for a workspace of that size.
 int ds_ld_for(int32_t S) { return (S + 255) / 256 * 256; }
 size_t bwd_ds_bytes(int32_t dtype, int32_t B, int32_t S, int32_t H) {
+    if (dtype == FA_DTYPE_F32) {
+        if (S > (1 << 22)) return 0;  // as the call itself; keeps the products below in 64 bits
+        const size_t nb = (size_t)(S + 31) / 32;
+        const size_t head = nb * nb * 4096, heads = (size_t)B * (size_t)H;
+        return heads > (size_t)FA_BWD_DS_MAX_BYTES / head ? 0 : heads * head;
+    }
     if (dtype != FA_DTYPE_BF16 || split_for(dtype, B, S, H) > 1 || fa::attn_waves(B, H, S) != 8) return 0;
     const int64_t head = (int64_t)(S + 31) / 32 * 32 * ds_ld_for(S) * 2;
     if (head >= (int64_t(1) << 32)) return 0;
@@ -206,8 +213,14 @@ size_t bwd_ds_bytes(int32_t dtype, int32_t B, int32_t S, int32_t H) {
     return bytes > (size_t)FA_BWD_DS_MAX_BYTES ? 0 : bytes;
 }
 
-size_t bwd_workspace(int32_t dtype, int32_t B, int32_t S, int32_t H, int32_t D) {
+size_t bwd_ds_workspace(int32_t dtype, int32_t B, int32_t S, int32_t H, int32_t D) {
     return bwd_min_workspace(dtype, B, S, H, D) + bwd_ds_bytes(dtype, B, S, H);
+}
+
+// What a caller that asks no further is told: f32 calls keep their rows only
+// (their dS is twice bf16's size), bf16 ones get their dS where it pays.
+size_t bwd_workspace(int32_t dtype, int32_t B, int32_t S, int32_t H, int32_t D) {
+    return dtype == FA_DTYPE_F32 ? bwd_min_workspace(dtype, B, S, H, D) : bwd_ds_workspace(dtype, B, S, H, D);
 }
 
 // forward workspace of a split call: O partials [split][B,H,S][D] f32, then
@@ -313,6 +326,11 @@ size_t fa_attn_bwd_workspace_size(const fa_attn_bwd_args *a) {
 size_t fa_attn_bwd_min_workspace_size(const fa_attn_bwd_args *a) {
     if (!a || a->batch < 1 || a->seq < 1 || a->heads < 1 || (a->head_dim != 64 && a->head_dim != 128)) return 0;
     return bwd_min_workspace(a->dtype, a->batch, a->seq, a->heads, a->head_dim);
+}
+
+size_t fa_attn_bwd_ds_workspace_size(const fa_attn_bwd_args *a) {
+    if (!a || a->batch < 1 || a->seq < 1 || a->heads < 1 || (a->head_dim != 64 && a->head_dim != 128)) return 0;
+    return bwd_ds_workspace(a->dtype, a->batch, a->seq, a->heads, a->head_dim);
 }
 
 fa_status fa_attn_bwd(const fa_attn_bwd_args *a, void *stream) {

@@ -72,6 +72,8 @@ int attn_split(int B, int H, int S);
 // f32 elements of the split partials per gradient or O (split * B*H*S*D).
 size_t attn_split_elems(int B, int H, int S, int D, int split);
 hipError_t launch_attn_bwd_f32(const AttnBwdParams &p, int D, int phase, hipStream_t s);
+// the f32 backward's phase 1 (attn_bwd.hip)
+hipError_t launch_attn_bwd_delta_f32(const AttnBwdParams &p, int D, hipStream_t s);
 
 // CU count of the current device (cached per device; 256 if unknown).
 int device_cu_count();

@@ -128,7 +128,7 @@ def attn_bwd_workspace_bytes(B: int, S: int, H: int, D: int, dtype=torch.bfloat1
     or, with minimum, the least fa_attn_bwd accepts (dQ recomputes S and dP).
     Both give the same bits."""
     ba = _abi.AttnBwdArgs(dtype=_dtype_code(torch.empty(0, dtype=dtype)), batch=B, seq=S, heads=H, head_dim=D)
-    f = lib().fa_attn_bwd_min_workspace_size if minimum else lib().fa_attn_bwd_workspace_size
+    f = lib().fa_attn_bwd_min_workspace_size if minimum else lib().fa_attn_bwd_ds_workspace_size
     return int(f(ctypes.byref(ba)))
 
 
@@ -187,7 +187,7 @@ def attn_bwd(q, k, v, o, dout, lse, scale: Optional[float] = None, key_keep=None
     # a given workspace of at least the minimum is used as it is (below the
     # full size: dQ recomputes S and dP); none gets the full size (dQ reads
     # the dK/dV kernel's stored dS)
-    need = lib().fa_attn_bwd_workspace_size(ctypes.byref(a))
+    need = lib().fa_attn_bwd_ds_workspace_size(ctypes.byref(a))
     least = lib().fa_attn_bwd_min_workspace_size(ctypes.byref(a))
     if workspace is None or workspace.numel() * workspace.element_size() < least:
         if workspace is not None and phases is not None:

@@ -156,6 +156,16 @@ size_t fa_attn_bwd_workspace_size(const fa_attn_bwd_args *args);
  * counterpart. */
 size_t fa_attn_bwd_min_workspace_size(const fa_attn_bwd_args *args);
 
+/* The workspace with which fa_attn_bwd stores dS wherever this build can (0 on
+ * bad args): fa_attn_bwd_workspace_size for bf16; for f32 that plus the f32 dS
+ * of every (key, query) pair ([B*H][seq][seq], both rounded up to 32; nothing
+ * past FA_BWD_DS_MAX_BYTES of it).  An f32 fa_attn_bwd given this much forms
+ * dQ from the stored dS, with the bits of the recomputing dQ; less (down to
+ * the minimum), the separate phases and fa_attn_bwd_noalloc recompute it, so
+ * the f32 phases stay independent of each other with any workspace.  No
+ * reference counterpart. */
+size_t fa_attn_bwd_ds_workspace_size(const fa_attn_bwd_args *args);
+
 /* dQ, dK, dV of the forward above: P is recomputed from Q, K and the saved
  * LSE; dS = P * (dP - rowsum(dO * O)) * scale; dQ = dS K, dK = dS^T Q,
  * dV = P^T dO, f32 accumulation, deterministic (no atomics).  For bf16 with
