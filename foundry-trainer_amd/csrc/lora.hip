@@ -5,29 +5,30 @@
 // produce its gradients.
 //
 //   rowdot  out[n][j] = s * sum_k X[n][k] W[j][k]      (x A^T, and dy B as
-//           dy (B^T)^T): a skinny GEMM.  bf16 (lora_rowdot16_kernel): 1, 2
-//           or 4 16-row slabs per 8-wave workgroup (chosen per call from the
-//           grid's fit to the CUs) on v_mfma_f32_16x16x32_bf16, each wave's
+//           dy (B^T)^T): a skinny GEMM (lora_rowdot16_kernel): 1, 2 or 4
+//           16-row slabs per 8-wave workgroup (chosen per call from the grid's
+//           fit to the CUs) on the 16x16 MFMA of the storage type, each wave's
 //           k-steps of X and W staged in its own LDS region by DMA in
-//           row-segment lane order and read back in operand order.  f32 (the
-//           parity path): one wave per 32 rows, operands from global memory.
+//           row-segment lane order and read back in operand order.
 //           HBM-bound: one read of X.
 //   expand  Y[n][c] += s * sum_j U[n][j] Wt[c][j]       (y += s u B^T, and
 //           dx += du A).  bf16 (lora_expand_mfma_kernel): one wave per 32
 //           rows x 64 columns on v_mfma_f32_32x32x16_bf16, the result
 //           transposed through LDS so Y is updated with 16-byte accesses.  f32
-//           (the parity path): one thread per output column and row phase,
-//           Wt rows staged in LDS.  HBM-bound: one read and one write of Y.
+//           (lora_expand_f32_kernel): 4 columns of W per lane in registers,
+//           waves walking rows.  HBM-bound: one read and one write of Y.
 //   colsum  out[j][c] = s * sum_n U[n][j] X[n][c]      (dB^T = s u^T dy and
-//           dA = du^T x).  bf16: a skinny MFMA GEMM, X^T (by transpose reads
-//           of 32-token x 128-column tiles streamed into LDS) times U^T (read
-//           the same way from a 32- or 64-column tile of U's rows streamed
-//           beside them, or from a staged fragment-major copy when U is not
-//           16-byte aligned), split over tokens; the splits are summed in a
-//           fixed order by a second kernel — deterministic, no atomics.  One
-//           set of launches serves up to 16 products of any token counts.
-//           f32 (the parity path): each workgroup owns 64 columns and sweeps
-//           all rows in a fixed order.
+//           dA = du^T x), split over tokens, the splits summed in a fixed
+//           order by a second kernel -- deterministic, no atomics.  bf16: X^T
+//           (by transpose reads of 32-token x 128-column tiles streamed into
+//           LDS) times U^T (read the same way from a 32- or 64-column tile of
+//           U's rows streamed beside them, or from a staged fragment-major
+//           copy when U is not 16-byte aligned); one set of launches serves up
+//           to 16 products of any token counts.  f32: both operands straight
+//           from memory into registers, both of an adapter's products in one
+//           grid.
+// The general f32 kernels (lora_rowdot_kernel, lora_expand_kernel,
+// lora_colsum_kernel) serve widths and strides the others do not address.
 #include <type_traits>
 
 #include "fa_device.hpp"
@@ -38,10 +39,11 @@ namespace fa {
 namespace {
 
 // ---- rowdot -------------------------------------------------------------
-// X: [N, K] (ldx), W: [R, K] contiguous, out: f32 [N, R] (ldo), R <= 32.
-template <typename T>
-__global__ __launch_bounds__(256) void lora_rowdot_kernel(const T *__restrict__ X, int64_t ldx,
-                                                          const T *__restrict__ W, float *out,
+// f32, general: X: [N, K] (ldx), W: [R, K] contiguous, out: f32 [N, R] (ldo),
+// R <= 32.  Serves what lora_rowdot16_kernel does not address: K not a
+// multiple of 4 (rows of W off 16-byte alignment) and spans past 32 bits.
+__global__ __launch_bounds__(256) void lora_rowdot_kernel(const float *__restrict__ X, int64_t ldx,
+                                                          const float *__restrict__ W, float *out,
                                                           int64_t ldo, int N, int K, int R,
                                                           float s) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -52,23 +54,12 @@ __global__ __launch_bounds__(256) void lora_rowdot_kernel(const T *__restrict__ 
     f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    if constexpr (sizeof(T) == 2) {
-        const bool xin = xr < N, win = n < R;
-        const bf16 *xp = reinterpret_cast<const bf16 *>(X) + (int64_t)xr * ldx + g * 8;
-        const bf16 *wp = reinterpret_cast<const bf16 *>(W) + (int64_t)n * K + g * 8;
-        for (int k0 = 0; k0 < K; k0 += 16) {
-            const bf16x8 a = as_bf16x8(xin ? ld_global_16(xp + k0) : u32x4{0, 0, 0, 0});
-            const bf16x8 b = as_bf16x8(win ? ld_global_16(wp + k0) : u32x4{0, 0, 0, 0});
-            acc = mfma_32x32x16(a, b, acc);
-        }
-    } else {
-        const float *xp = reinterpret_cast<const float *>(X) + (int64_t)xr * ldx;
-        const float *wp = reinterpret_cast<const float *>(W) + (int64_t)n * K;
-        for (int k0 = 0; k0 < K; k0 += 2) {
-            const float a = xr < N ? xp[k0 + g] : 0.f;
-            const float b = n < R ? wp[k0 + g] : 0.f;
-            acc = mfma_32x32x2_f32(a, b, acc);
-        }
+    const float *xp = X + (int64_t)xr * ldx;
+    const float *wp = W + (int64_t)n * K;
+    for (int k0 = 0; k0 < K; k0 += 2) {
+        const float a = xr < N ? xp[k0 + g] : 0.f;
+        const float b = n < R ? wp[k0 + g] : 0.f;
+        acc = mfma_32x32x2_f32(a, b, acc);
     }
     // acc element r: row row0 + acc_row(r), column j = n
     if (n < R)
@@ -79,21 +70,22 @@ __global__ __launch_bounds__(256) void lora_rowdot_kernel(const T *__restrict__ 
         }
 }
 
-// ---- expand -------------------------------------------------------------
-// Y[n][c] += s * sum_j U[n][j] * Wt[c][j];  U f32 [N, R] (ldu), Wt [C, R]
-// contiguous, Y [N, C] (ldy).  Block = 64 columns x 4 row phases; the 64 Wt
-// rows are staged in LDS, U rows are broadcast reads.
-template <typename T>
+// ---- expand, f32 --------------------------------------------------------
+// Y[n][c] += s * sum_j U[n][j] * W(c, j), W(c, j) at c * ws_c + j * ws_j, U f32
+// [N, R] (ldu), Y [N, C] (ldy).
+//
+// General: block = 64 columns x 4 row phases; the 64 columns of W are staged
+// in LDS, U rows are broadcast reads.
 __global__ __launch_bounds__(256) void lora_expand_kernel(const float *__restrict__ U, int64_t ldu,
-                                                          const T *__restrict__ Wt, T *Y,
-                                                          int64_t ldy, int N, int C, int R,
+                                                          const float *__restrict__ W, int64_t ws_c, int64_t ws_j,
+                                                          float *Y, int64_t ldy, int N, int C, int R,
                                                           float s, int rows_per_block) {
     __shared__ float wsh[64][33];
     const int cl = threadIdx.x & 63, ph = threadIdx.x >> 6;
     const int c0 = blockIdx.x * 64;
     for (int e = threadIdx.x; e < 64 * R; e += 256) {
         const int cc = e / R, j = e % R;
-        wsh[cc][j] = c0 + cc < C ? (float)Wt[(int64_t)(c0 + cc) * R + j] : 0.f;
+        wsh[cc][j] = c0 + cc < C ? W[(c0 + cc) * ws_c + j * ws_j] : 0.f;
     }
     __syncthreads();
     const int col = c0 + cl;
@@ -104,14 +96,88 @@ __global__ __launch_bounds__(256) void lora_expand_kernel(const float *__restric
         const float *u = U + (int64_t)row * ldu;
         float acc = 0.f;
         for (int j = 0; j < R; ++j) acc += u[j] * wsh[cl][j];
-        T *y = Y + (int64_t)row * ldy + col;
-        *y = (T)((float)*y + s * acc);
+        float *y = Y + (int64_t)row * ldy + col;
+        *y = *y + s * acc;
     }
 }
 
-// ---- rowdot / expand, bf16 (MFMA) ---------------------------------------
+// Y's rows 16-byte aligned and C % 4 == 0: a lane owns 4 columns, whose W
+// values stay in registers while its wave walks rows, so a wave reads and
+// writes 1 KiB of one row per access and U's row (the same for every lane)
+// comes through scalar registers.  Bound by Y's read and write (1536 x 3072 at
+// r 16: 20.6 -> 10.5 us against a column per thread, 3.6 TB/s).  The sum runs
+// over j in order, as the general kernel's.  RP: R rounded up to 16 or 32, the
+// values past R zero on both sides; EXACT: R == RP.  JROWS: W is [R][C] (else
+// [C][R]).  W's 256 columns go through LDS, [j][column] (rows padded to 260:
+// the fill from [C][R] hits 64 banks), so that either layout is read
+// contiguously; its loads and the first rows of Y go out before any is used.
+// Bounds are the buffer descriptors': past them loads give zero and stores are
+// dropped, so nothing in the loop branches.
+template <int RP, bool EXACT, bool JROWS>
+__global__ __launch_bounds__(256) void lora_expand_f32_kernel(const float *__restrict__ U, int64_t ldu,
+                                                              const float *__restrict__ W, float *Y, int64_t ldy,
+                                                              int N, int C, int R, float s, int rows_per_wave) {
+    constexpr int LDW = 260;
+    constexpr int RB = 4;  // rows in flight
+    __shared__ __align__(16) float wsh[RP * LDW];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int cb = blockIdx.x * 256, col = cb + lane * 4;
+    const int n0 = (blockIdx.y * 4 + wave) * rows_per_wave, rows = min(N - n0, rows_per_wave);
+    const __amdgpu_buffer_rsrc_t yrs =
+        make_rsrc(Y + (int64_t)n0 * ldy, rows > 0 ? (uint32_t)(((rows - 1) * ldy + C) * 4) : 0u);
+    const __amdgpu_buffer_rsrc_t wrs = make_rsrc(W, (uint32_t)((int64_t)R * C * 4));
+    const uint32_t yrow = (uint32_t)(ldy * 4);
+    f32x4 y[RB];
+    auto load = [&](int row) {
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+            y[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(yrs, col * 4, (row + i) * yrow, 0));
+    };
+    load(0);
+    float wv[RP];
+#pragma unroll
+    for (int i = 0; i < RP; ++i) {
+        const uint32_t e = JROWS ? (uint32_t)i * (uint32_t)C + cb + tid : (uint32_t)cb * (uint32_t)R + i * 256 + tid;
+        wv[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(wrs, e * 4, 0, 0));
+    }
+#pragma unroll
+    for (int i = 0; i < RP; ++i) {
+        const int e = i * 256 + tid, cc = JROWS ? tid : EXACT ? e / RP : e / R, j = JROWS ? i : e - cc * (EXACT ? RP : R);
+        if (EXACT || i < R) wsh[j * LDW + cc] = wv[i];
+    }
+    __syncthreads();
+    if (col >= C) return;
+    f32x4 w[RP];
+#pragma unroll
+    for (int j = 0; j < RP; ++j)
+        w[j] = EXACT || j < R ? *reinterpret_cast<const f32x4 *>(wsh + j * LDW + lane * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int row = 0; row < rows; row += RB) {
+        f32x4 out[RB];
+#pragma unroll
+        for (int i = 0; i < RB; ++i) out[i] = y[i];
+        load(row + RB);
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            const float *u = U + (int64_t)min(n0 + row + i, N - 1) * ldu;
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < RP; ++j) {
+                const float uj = EXACT ? u[j] : j < R ? u[min(j, R - 1)] : 0.f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] += uj * w[j][e];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[i][e] += s * acc[e];
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, out[i]), yrs, col * 4, (row + i) * yrow, 0);
+        }
+    }
+}
+
+// ---- rowdot (MFMA), expand bf16 (MFMA) ----------------------------------
 // rowdot: out[n][j] = s * sum_k X[n][k] W[j][k], R <= 16 * NT.  A workgroup
-// of 8 waves owns 16 rows; wave w takes k-steps (32 wide) w, w + 8, ..., and
+// of 8 waves owns 16 rows; wave w takes k-steps (64 bytes of a row: 32 bf16 or
+// 16 f32 columns) w, w + 8, ..., and
 // the 8 partial tiles are summed in LDS in a fixed order (deterministic, no
 // workspace).
 //
@@ -127,14 +193,18 @@ __global__ __launch_bounds__(256) void lora_expand_kernel(const float *__restric
 // G k-steps per stage, two stages per wave in flight; no barrier inside the
 // loop (the regions are private).  Rows >= N and j >= R load from a clamped (valid) row:
 // output element (n, j) depends on row n of X and row j of W only, and those
-// outputs are not stored.  K % 32 == 16 leaves a half k-step whose upper 16
-// columns are zeroed in the operand.
-// One k-step per stage: two k-steps per stage (twice the LDS) was no faster
-// alone and slower in the c4 step, where a workgroup's LDS decides whether it
-// can share a CU with the other stream's kernels.
-template <int NT, int MT = 1>
+// outputs are not stored.  A last k-step cut short by K (K is a multiple of
+// a 16-byte chunk) has its chunks past K zeroed in the X operand.
+// One k-step per stage in bf16: two k-steps per stage (twice the LDS) was no
+// faster alone and slower in the c4 step, where a workgroup's LDS decides
+// whether it can share a CU with the other stream's kernels.  f32 rows have
+// twice the k-steps: two per stage there.
+// f32 operands are chunks of 4 columns, fed to v_mfma_f32_16x16x4_f32 one
+// column of each lane's chunk at a time.  Replacing one wave per 32 rows with
+// 4-byte loads, 1536 x 3072 at r 16: 283 -> 10 us.
+template <typename T, int NT, int MT = 1>
 struct RowdotStage {
-    static constexpr int G = 1;                        // k-steps per stage
+    static constexpr int G = sizeof(T) == 4 && MT < 4 ? 2 : 1;  // k-steps per stage (two stages within 160 KiB)
     static constexpr int STEP = 1024 * (MT + NT);      // LDS bytes per k-step: MT X slabs, then NT W tiles
     static constexpr int WAVE = G * STEP;              // one wave's stage
     static constexpr int BYTES = 8 * WAVE;             // the workgroup's stage
@@ -143,11 +213,12 @@ struct RowdotStage {
 // MT: 16-row slabs per workgroup.  Each k-step's W tiles are then read once
 // for MT slabs of X; at rank 48 the W bytes (from L2) outweigh X's three to
 // one for a single slab.
-template <int NT, typename TO, int MT = 1>
-__global__ __launch_bounds__(512) void lora_rowdot16_kernel(const bf16 *__restrict__ X, int64_t ldx,
-                                                            const bf16 *__restrict__ W, TO *out, int64_t ldo,
+template <typename T, int NT, typename TO, int MT = 1>
+__global__ __launch_bounds__(512) void lora_rowdot16_kernel(const T *__restrict__ X, int64_t ldx,
+                                                            const T *__restrict__ W, TO *out, int64_t ldo,
                                                             int N, int K, int R, float s) {
-    using RS = RowdotStage<NT, MT>;
+    using RS = RowdotStage<T, NT, MT>;
+    constexpr int E = sizeof(T), CE = 16 / E, KE = 64 / E;  // bytes per element, elements per chunk and per k-step
     constexpr int G = RS::G;
     // two distinct LDS objects: the compiler then tells the DMA into one
     // stage from the reads of the other
@@ -161,24 +232,24 @@ __global__ __launch_bounds__(512) void lora_rowdot16_kernel(const bf16 *__restri
     const int row0 = blockIdx.x * 16 * MT;
 
     // DMA source offsets: lane 4 r + p fetches chunk p ^ ((r / 4) % 4) of row
-    // r of a 16-row, 32-column k-step (the k-step itself goes in soffset)
+    // r of a 16-row, 64-byte-wide k-step (the k-step itself goes in soffset)
     const int r = lane >> 2, c = (lane & 3) ^ ((r >> 2) & 3);
     const int xrows = min(16 * MT, N - row0);
     const __amdgpu_buffer_rsrc_t xrs =
-        make_rsrc(X + (int64_t)row0 * ldx, (uint32_t)(((int64_t)(xrows - 1) * ldx + K) * 2));
-    const __amdgpu_buffer_rsrc_t wrs = make_rsrc(W, (uint32_t)((int64_t)R * K * 2));
+        make_rsrc(X + (int64_t)row0 * ldx, (uint32_t)(((int64_t)(xrows - 1) * ldx + K) * E));
+    const __amdgpu_buffer_rsrc_t wrs = make_rsrc(W, (uint32_t)((int64_t)R * K * E));
     uint32_t xvo[MT];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) xvo[mt] = (uint32_t)((min(mt * 16 + r, xrows - 1) * ldx + c * 8) * 2);
+    for (int mt = 0; mt < MT; ++mt) xvo[mt] = (uint32_t)((min(mt * 16 + r, xrows - 1) * ldx + c * CE) * E);
     uint32_t wvo[NT];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) wvo[t] = (uint32_t)((min(t * 16 + r, R - 1) * (int64_t)K + c * 8) * 2);
+    for (int t = 0; t < NT; ++t) wvo[t] = (uint32_t)((min(t * 16 + r, R - 1) * (int64_t)K + c * CE) * E);
     // operand reads: lane (m, q) takes chunk q of row m
     const int rd = m * 64 + ((q ^ ((m >> 2) & 3)) << 4);
 
-    const int nks = (K + 31) / 32;                               // k-steps, the last maybe half
+    const int nks = (K + KE - 1) / KE;                           // k-steps, the last maybe cut short
     const int J = nks > wave ? (nks - wave + 7) / 8 : 0;         // this wave's k-steps
-    const bool half = K % 32 != 0;
+    const int tail = K % KE != 0 ? K % KE / CE : 4;              // chunks of the last k-step
     // stage of k-steps j0 .. j0+G-1 of this wave into dst; past J it loads a
     // clamped (valid) k-step that is never read, so every stage issues the
     // same G (1 + NT) loads and the waits can count them
@@ -212,9 +283,17 @@ __global__ __launch_bounds__(512) void lora_rowdot16_kernel(const bf16 *__restri
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
                     u32x4 a = ld_lds_16(d + g * RS::STEP + 1024 * mt, rd);
-                    if (half && wave + 8 * (j0 + g) == nks - 1 && q >= 2) a = zero;  // columns past K
+                    if (tail < 4 && wave + 8 * (j0 + g) == nks - 1 && q >= tail) a = zero;  // columns past K
 #pragma unroll
-                    for (int t = 0; t < NT; ++t) acc[mt][t] = mfma_16x16x32(as_bf16x8(a), as_bf16x8(wf[t]), acc[mt][t]);
+                    for (int t = 0; t < NT; ++t) {
+                        if constexpr (E == 2) {
+                            acc[mt][t] = mfma_16x16x32(as_bf16x8(a), as_bf16x8(wf[t]), acc[mt][t]);
+                        } else {
+                            const f32x4 af = __builtin_bit_cast(f32x4, a), bf = __builtin_bit_cast(f32x4, wf[t]);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) acc[mt][t] = mfma_16x16x4_f32(af[e], bf[e], acc[mt][t]);
+                        }
+                    }
                 }
             }
     };
@@ -395,16 +474,16 @@ __global__ __launch_bounds__(256) void lora_expand_mfma_kernel(const TU *__restr
     }
 }
 
-// ---- colsum -------------------------------------------------------------
+// ---- colsum, f32 ---------------------------------------------------------
 // out[j][c] = s * sum_n U[n][j] * X[n][c]  (U f32 [N, R], X [N, C] ldx).
 // Written to out at (j * os_j + c * os_c) so the same kernel yields dA [R, K]
 // (os_j = K, os_c = 1) and dB [M, R] (os_j = 1, os_c = R).
-// Block: 64 columns x 4 row-phases; each thread accumulates R partial sums
-// for one column over rows phase, phase+4, ..., then the 4 phases are summed
-// in a fixed order.
-template <typename T>
+//
+// General (16 rows of X spanning 4 GiB or more): 64 columns x 4 row phases per
+// block; each thread accumulates R partial sums for one column over rows
+// phase, phase+4, ..., then the 4 phases are summed in a fixed order.
 __global__ __launch_bounds__(256) void lora_colsum_kernel(const float *__restrict__ U, int64_t ldu,
-                                                          const T *__restrict__ X, int64_t ldx,
+                                                          const float *__restrict__ X, int64_t ldx,
                                                           float *out, int64_t os_j, int64_t os_c,
                                                           int N, int C, int R, float s) {
     __shared__ float part[4][64][33];
@@ -415,7 +494,7 @@ __global__ __launch_bounds__(256) void lora_colsum_kernel(const float *__restric
     for (int j = 0; j < 32; ++j) acc[j] = 0.f;
     if (col < C) {
         for (int row = ph; row < N; row += 4) {
-            const float xv = (float)X[(int64_t)row * ldx + col];
+            const float xv = X[(int64_t)row * ldx + col];
             const float *u = U + (int64_t)row * ldu;
 #pragma unroll
             for (int j = 0; j < 32; ++j)
@@ -429,6 +508,107 @@ __global__ __launch_bounds__(256) void lora_colsum_kernel(const float *__restric
         for (int j = 0; j < R; ++j)
             out[j * os_j + (int64_t)col * os_c] =
                 s * (((part[0][cl][j] + part[1][cl][j]) + part[2][cl][j]) + part[3][cl][j]);
+}
+
+// Both gradients of an adapter (dB from u and dy, dA from du and x) in one
+// grid, HBM-bound: one read of X each.  A workgroup owns 128 columns of a
+// product over one token split; its 4 waves take every fourth 16-token block
+// of it.  Lane (n, g) holds columns 4n .. +3 of token 2i + g in one 16-byte
+// load (512 contiguous bytes per token) and U's column n of that token: X^T
+// and U as the operands of four v_mfma_f32_32x32x2_f32, one per column
+// residue, a block's loads in flight while the block before is multiplied.
+// The waves' sums are added in LDS, the splits by the reduce kernel, both in
+// a fixed order.  1536 x 3072 at r 16: 466 -> 8 us per product, against 64
+// columns per workgroup over all tokens.
+struct CsItem {
+    const float *u;
+    int64_t ldu;
+    const float *x;
+    int64_t ldx;
+    float *out;
+    int64_t os_j, os_c;
+    float *part;  // [splits][C][R]; unused when splits is 1
+    float s;
+    int C, splits, chunk, wg0;  // tokens per split (a multiple of 16); the product's first workgroup
+};
+struct CsPair {
+    CsItem p[2];
+    int N, R;
+};
+
+__global__ __launch_bounds__(256) void lora_colsum_f32_kernel(CsPair g2) {
+    __shared__ float part[4][2][16][64];  // two column residues at a time
+    const CsItem &q = g2.p[(int)blockIdx.x >= g2.p[1].wg0 ? 1 : 0];
+    const int lane = threadIdx.x & 63, n = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int R = g2.R, C = q.C;
+    const int tiles = (C + 127) / 128;
+    const int wi = (int)blockIdx.x - q.wg0, sp = wi / tiles, c0 = (wi - sp * tiles) * 128;
+    const int t1 = min(g2.N, (sp + 1) * q.chunk);
+    f32x16 acc[4];
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
+    struct Operands {
+        f32x4 x[8];
+        float u[8];
+    };
+    // Tokens t .. t+15 (rows past t1, and everything past the matrices' last
+    // element, read as zero); columns past C and j past R hold other rows'
+    // values and reach outputs that are not stored only.
+    const uint32_t xr = (uint32_t)(q.ldx * 4), ur = (uint32_t)(q.ldu * 4);
+    auto load = [&](int t, Operands &o) {
+        const int rows = min(16, t1 - t);
+        const __amdgpu_buffer_rsrc_t xrs =
+            make_rsrc(q.x + (int64_t)t * q.ldx + c0, rows > 0 ? (uint32_t)(((rows - 1) * q.ldx + (C - c0)) * 4) : 0u);
+        const __amdgpu_buffer_rsrc_t urs =
+            make_rsrc(q.u + (int64_t)t * q.ldu, rows > 0 ? (uint32_t)(((rows - 1) * q.ldu + R) * 4) : 0u);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            o.x[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, g * xr + n * 16, 2 * i * xr, 0));
+            o.u[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(urs, g * ur + n * 4, 2 * i * ur, 0));
+        }
+    };
+    auto step = [&](int next, const Operands &o, Operands &nx) {
+        load(next, nx);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) acc[dt] = mfma_32x32x2_f32(o.x[i][dt], o.u[i], acc[dt]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Operands a, b;
+    int t = sp * q.chunk + wave * 16;
+    load(t, a);
+    for (; t < t1; t += 128) {
+        step(t + 64, a, b);
+        step(t + 128, b, a);  // past t1: zeros
+    }
+    // element r of acc[dt]: column c0 + 4 acc_row(r) + dt, j = n
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        __syncthreads();
+#pragma unroll
+        for (int d = 0; d < 2; ++d)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) part[wave][d][r][lane] = acc[2 * h + d][r];
+        __syncthreads();
+#pragma unroll
+        for (int d = 0; d < 2; ++d)
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) {
+                const int r = wave * 4 + rr, c = c0 + 4 * acc_row(r, lane) + 2 * h + d;
+                const float v = ((part[0][d][r][lane] + part[1][d][r][lane]) + part[2][d][r][lane]) + part[3][d][r][lane];
+                if (n < R && c < C) {
+                    if (q.splits == 1)
+                        q.out[n * q.os_j + (int64_t)c * q.os_c] = q.s * v;
+                    else
+                        q.part[((int64_t)sp * C + c) * R + n] = v;
+                }
+            }
+    }
 }
 
 // ---- colsum, bf16 (MFMA) ------------------------------------------------
@@ -450,90 +630,12 @@ __device__ __forceinline__ void ut_frag_coords(int64_t e, int npad, int &j, int 
     const int q = p & 15;
     n = (p >> 4) * 16 + ((q & 4) ? 8 : 0) + ((q & 8) ? 4 : 0) + (q & 3);
 }
-template <typename TU>
-__global__ void lora_ut_kernel(const TU *__restrict__ U, int64_t ldu, bf16 *ut, int N, int R, int npad) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= (int64_t)32 * npad) return;
-    int j, n;
-    ut_frag_coords(e, npad, j, n);
-    ut[e] = j < R && n < N ? (bf16)U[(int64_t)n * ldu + j] : (bf16)0.f;
-}
-
 constexpr int kCsCols = 128;  // columns per workgroup (4 waves x 32)
 // Tokens per LDS stage.  32 rather than 64: 24 KiB of LDS per workgroup
 // (two stages of X and U) lets six workgroups share a CU instead of three;
 // the c4 step's 12 gradient products 41.0 -> 38.4 us, the single block's
 // four 110.3 -> 103.8 us, same bits (a 4-product q/k/v set 23.7 -> 24.9 us).
 constexpr int kCsRows = 32;
-
-// Workgroup (column tile ct, token split sp): part[sp][c][j] = sum over the
-// split's tokens of X[n][c] U[n][j], for the tile's 128 columns and j < 32.
-__global__ __launch_bounds__(256) void lora_colsum_mfma_kernel(const bf16 *__restrict__ X, int64_t ldx,
-                                                               const bf16 *__restrict__ ut, int npad,
-                                                               float *part, int N, int C, int chunk) {
-    using T = LdsTile<128, kCsRows>;
-    constexpr int WI = T::WAVE_INSTS / 4;
-    __shared__ __align__(16) char st0[T::BYTES], st1[T::BYTES];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n = lane & 31;
-    const int c0 = blockIdx.x * kCsCols;
-    const int t_begin = blockIdx.y * chunk, t_end = min(t_begin + chunk, npad);
-    // rows >= N (and, in the last row, columns >= C) read as zero
-    const __amdgpu_buffer_rsrc_t xrs = make_rsrc(X + c0, (uint32_t)(((int64_t)(N - 1) * ldx + (C - c0)) * 2));
-    const uint32_t xvo = tile_src_off<128>(wave, lane, ldx);
-    const uint32_t row_step = tile_inst_row_step<128>(ldx);
-    const uint32_t stage_step = (uint32_t)(kCsRows * ldx * 2);
-    auto issue = [&](int t0, char *dst) {
-#pragma unroll
-        for (int i = 0; i < WI; ++i)
-            buffer_to_lds_16(xrs, dst + (i * 4 + wave) * 1024, xvo, (uint32_t)(t0 / kCsRows) * stage_step + i * row_step);
-    };
-    uint32_t coff[4];
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) coff[dt] = col_frag_off<128>(0, 0, dt, lane);
-    const bf16 *ub = ut + lane * 8;  // fragment-major: 512 values per 16-token step
-    f32x16 acc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    // a stage's U^T fragments are loaded before the next stage's DMA, so that
-    // waiting for them leaves that DMA in flight (in-order completion)
-    constexpr int KS = kCsRows / 16;
-    auto loadu = [&](int t0, bf16x8 (&b)[KS]) {
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) b[ks] = as_bf16x8(ld_global_16(ub + ((t0 >> 4) + ks) * 512));
-    };
-    auto stage = [&](const char *tile, const bf16x8 (&b)[KS]) {
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const bf16x8 a = lds_read_col_frag(tile, coff[wave] + ks * 16 * T::ROWB,
-                                               col_frag_hi8<128>(coff, wave) + ks * 16 * T::ROWB);
-            acc = mfma_32x32x16(a, b[ks], acc);
-        }
-    };
-    bf16x8 bu[KS];
-    issue(t_begin, st0);
-    for (int t0 = t_begin; t0 < t_end; t0 += 2 * kCsRows) {
-        barrier_keep_dma<0>();
-        loadu(t0, bu);
-        if (t0 + kCsRows < t_end) issue(t0 + kCsRows, st1);
-        stage(st0, bu);
-        if (t0 + kCsRows < t_end) {
-            barrier_keep_dma<0>();
-            loadu(t0 + kCsRows, bu);
-            if (t0 + 2 * kCsRows < t_end) issue(t0 + 2 * kCsRows, st0);
-            stage(st1, bu);
-        }
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    // acc element r: column c0 + wave*32 + acc_row(r, lane), j = n
-    float *pp = part + (int64_t)blockIdx.y * C * 32;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int c = c0 + wave * 32 + acc_row(r, lane);
-        if (c < C) pp[(int64_t)c * 32 + n] = acc[r];
-    }
-}
 
 // sum_sp p[sp * stride] for sp = 0, 1, ..., n - 1, added in that order; the
 // loads go out eight at a time, so a thread waits for memory once per eight
@@ -552,23 +654,23 @@ __device__ __forceinline__ float sum_splits(const float *p, int64_t stride, int 
     return acc;
 }
 
-// out[j * os_j + c * os_c] = s * sum_sp part[sp][c][j] (fixed order), j < R.
-__global__ void lora_colsum_reduce_kernel(const float *__restrict__ part, float *out, int64_t os_j,
-                                          int64_t os_c, int C, int R, int splits, float s) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= (int64_t)C * 32) return;
-    const int c = (int)(e >> 5), j = (int)(e & 31);
-    if (j >= R) return;
-    out[j * os_j + (int64_t)c * os_c] = s * sum_splits(part + e, (int64_t)C * 32, splits);
+// f32: out[j * os_j + c * os_c] = s * sum_sp part[sp][c][j] (fixed order).
+__global__ void lora_colsum_reduce_f32_kernel(CsPair g2) {
+    const CsItem &q = g2.p[blockIdx.y];
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x, n = (int64_t)q.C * g2.R;
+    if (q.splits == 1 || e >= n) return;
+    const int c = (int)(e / g2.R), j = (int)(e - (int64_t)c * g2.R);
+    q.out[j * q.os_j + (int64_t)c * q.os_c] = q.s * sum_splits(q.part + e, n, q.splits);
 }
 
 // ---- colsum over several products in one set of launches -----------------
 // Products k = 0..count-1, each of its own token count N_k: out_k = s_k *
-// U_k^T X_k (or its transpose), U_k bf16 [N_k, R_k <= 64].  The same three steps as above,
-// each one launch for all products: U^T in operand order (rw = 32 or 64 rows),
-// split partials over [splits_k][C_k][rw] (R_k > 32: a second accumulator
-// over U^T rows 32..63 shares each X tile), fixed-order sum.  Per output the
-// arithmetic is that of the single-product kernels, so the same bits.
+// U_k^T X_k (or its transpose), U_k bf16 [N_k, R_k <= 64].  Three steps, each
+// one launch for all products: U^T in operand order (rw = 32 or 64 rows; only
+// for U that is not 16-byte aligned), split partials over [splits_k][C_k][rw]
+// (R_k > 32: a second accumulator over U^T rows 32..63 shares each X tile),
+// fixed-order sum.  A product's splits depend on its own N and C only, so its
+// bits do not depend on the others.
 constexpr int kGradMany = 16;
 struct GradProblem {
     const bf16 *u;
@@ -782,13 +884,32 @@ __global__ void lora_colsum_reduce_many_kernel(GradMany g) {
     q.out[j * q.os_j + (int64_t)c * q.os_c] = q.s * sum_splits(q.part + e, (int64_t)q.C * q.rw, q.splits);
 }
 
-// Small transpose [R][C] -> [C][R] (dtype).
+// What the backward's products read, in one launch: B^T [R][M] (the rowdot's
+// row operand), and for bf16 A^T [K][R] (the expand's operand, when dx is
+// wanted) and u rounded to bf16 rows of stride ldub (16-byte aligned, as the
+// colsum's DMA reads them; every product rounds u to bf16 anyway).
 template <typename T>
-__global__ void lora_transpose_kernel(const T *__restrict__ src, T *dst, int R, int C) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= (int64_t)R * C) return;
-    const int r = e / C, c = e % C;
-    dst[(int64_t)c * R + r] = src[e];
+struct BwdPrep {
+    const T *b, *a;
+    const float *u;
+    T *bt, *at;
+    bf16 *ub;
+    int M, K, N, R, ldub;
+    int wg_a, wg_u;  // first workgroups of the second and third part
+};
+template <typename T>
+__global__ __launch_bounds__(256) void lora_bwd_prep_kernel(BwdPrep<T> p) {
+    const int wg = (int)blockIdx.x;
+    if (wg < p.wg_a) {
+        const int64_t e = (int64_t)wg * 256 + threadIdx.x;  // of B^T: reads of one row are strided, writes contiguous
+        if (e < (int64_t)p.R * p.M) p.bt[e] = p.b[(e % p.M) * p.R + e / p.M];
+    } else if (wg < p.wg_u) {
+        const int64_t e = (int64_t)(wg - p.wg_a) * 256 + threadIdx.x;  // of A
+        if (e < (int64_t)p.R * p.K) p.at[(e % p.K) * p.R + e / p.K] = p.a[e];
+    } else {
+        const int64_t e = (int64_t)(wg - p.wg_u) * 256 + threadIdx.x;
+        if (e < (int64_t)p.N * p.R) p.ub[e / p.R * p.ldub + e % p.R] = f32_to_bf16(p.u[e]);
+    }
 }
 
 // 16-row slabs per rowdot workgroup, 1, 2 or 4.  A CU's LDS-DMA rate bounds
@@ -811,29 +932,41 @@ int rowdot_slabs(int N, int NT) {
     return best;
 }
 
-template <typename T>
-hipError_t rowdot(const T *X, int64_t ldx, const T *W, float *out, int64_t ldo, int N, int K,
-                  int R, float s, hipStream_t st) {
-    if constexpr (sizeof(T) == 2) {
-        auto go = [&](auto mtc) {
-            constexpr int MT = decltype(mtc)::value;
-            const dim3 grid((unsigned)((N + 16 * MT - 1) / (16 * MT))), block(512);
-            if (R <= 16)
-                hipLaunchKernelGGL((lora_rowdot16_kernel<1, float, MT>), grid, block, 0, st, X, ldx, W, out, ldo, N, K,
-                                   R, s);
-            else
-                hipLaunchKernelGGL((lora_rowdot16_kernel<2, float, MT>), grid, block, 0, st, X, ldx, W, out, ldo, N, K,
-                                   R, s);
+// R <= 64 (f32: 32): up to four 16-column tiles per workgroup (a stack of
+// adapters that share x, e.g. q/k/v, runs as one product)
+template <typename T, typename TO>
+hipError_t rowdot16(const T *X, int64_t ldx, const T *W, TO *out, int64_t ldo, int N, int K, int R, float s,
+                    hipStream_t st) {
+    auto go = [&](auto mtc) {
+        constexpr int MT = decltype(mtc)::value;
+        const dim3 grid((unsigned)((N + 16 * MT - 1) / (16 * MT))), block(512);
+        auto pick = [&](auto ntc) {
+            constexpr int NT = decltype(ntc)::value;
+            hipLaunchKernelGGL((lora_rowdot16_kernel<T, NT, TO, MT>), grid, block, 0, st, X, ldx, W, out, ldo, N, K, R,
+                               s);
         };
-        switch (rowdot_slabs(N, (R + 15) / 16)) {
-        case 1: go(std::integral_constant<int, 1>{}); break;
-        case 2: go(std::integral_constant<int, 2>{}); break;
-        default: go(std::integral_constant<int, 4>{}); break;
+        if (R <= 16) return pick(std::integral_constant<int, 1>{});
+        if (sizeof(T) == 4 || R <= 32) return pick(std::integral_constant<int, 2>{});
+        if constexpr (sizeof(T) == 2) {
+            if (R <= 48) return pick(std::integral_constant<int, 3>{});
+            return pick(std::integral_constant<int, 4>{});
         }
-    } else {
-        const dim3 grid((N + 127) / 128), block(256);
-        hipLaunchKernelGGL(lora_rowdot_kernel<T>, grid, block, 0, st, X, ldx, W, out, ldo, N, K, R, s);
+    };
+    switch (rowdot_slabs(N, (R + 15) / 16)) {
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    default: go(std::integral_constant<int, 4>{}); break;
     }
+    return hipGetLastError();
+}
+
+hipError_t rowdot(const float *X, int64_t ldx, const float *W, float *out, int64_t ldo, int N, int K, int R, float s,
+                  hipStream_t st) {
+    // 16-byte W rows, and 64 rows of X and all of W within 32-bit byte offsets
+    const int64_t xspan = (int64_t)63 * ldx + K, wspan = (int64_t)R * K;
+    if (K % 4 == 0 && xspan < (1 << 30) && wspan < (1 << 30))
+        return rowdot16<float, float>(X, ldx, W, out, ldo, N, K, R, s, st);
+    hipLaunchKernelGGL(lora_rowdot_kernel, dim3((N + 127) / 128), dim3(256), 0, st, X, ldx, W, out, ldo, N, K, R, s);
     return hipGetLastError();
 }
 
@@ -864,14 +997,39 @@ hipError_t expand_mfma(const TU *U, int64_t ldu, const bf16 *Wt, bf16 *Y, int64_
     return hipGetLastError();
 }
 
-template <typename T>
-hipError_t expand(const float *U, int64_t ldu, const T *Wt, T *Y, int64_t ldy, int N, int C,
-                  int R, float s, hipStream_t st) {
-    if constexpr (sizeof(T) == 2) return expand_mfma<float>(U, ldu, Wt, Y, ldy, N, C, R, s, st);
+// f32 Y += s * U W^T, W [C][R], or [R][C] with jrows.  Rows per wave: 16, fewer
+// where that would leave CUs without two workgroups.
+hipError_t expand_f32(const float *U, int64_t ldu, const float *W, bool jrows, float *Y, int64_t ldy, int N, int C,
+                      int R, float s, hipStream_t st) {
+    const int bx = (C + 255) / 256, cus = device_cu_count();
+    int rpw = 16;
+    while (rpw > 4 && (int64_t)bx * ((N + 4 * rpw - 1) / (4 * rpw)) < 2 * cus) rpw /= 2;
+    const dim3 grid((unsigned)bx, (unsigned)((N + 4 * rpw - 1) / (4 * rpw))), block(256);
+    // 16-byte rows; a wave's rows, and W, within 32-bit byte offsets
+    if (C % 4 == 0 && ldy % 4 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0 && ldy < (1 << 25) &&
+        (int64_t)R * C < (1 << 29) && grid.y <= 65535) {
+        auto go = [&](auto rp, auto exact) {
+            constexpr int RP = decltype(rp)::value;
+            constexpr bool EX = decltype(exact)::value;
+            if (jrows)
+                hipLaunchKernelGGL((lora_expand_f32_kernel<RP, EX, true>), grid, block, 0, st, U, ldu, W, Y, ldy, N, C,
+                                   R, s, rpw);
+            else
+                hipLaunchKernelGGL((lora_expand_f32_kernel<RP, EX, false>), grid, block, 0, st, U, ldu, W, Y, ldy, N,
+                                   C, R, s, rpw);
+        };
+        using R16 = std::integral_constant<int, 16>;
+        using R32 = std::integral_constant<int, 32>;
+        if (R == 16) go(R16{}, std::true_type{});
+        else if (R < 16) go(R16{}, std::false_type{});
+        else if (R == 32) go(R32{}, std::true_type{});
+        else go(R32{}, std::false_type{});
+        return hipGetLastError();
+    }
     const int rpb = 64;
-    const dim3 grid((C + 63) / 64, (N + rpb - 1) / rpb), block(256);
-    hipLaunchKernelGGL(lora_expand_kernel<T>, grid, block, 0, st, U, ldu, Wt, Y, ldy, N, C, R, s,
-                       rpb);
+    const dim3 ggrid((C + 63) / 64, (N + rpb - 1) / rpb);
+    hipLaunchKernelGGL(lora_expand_kernel, ggrid, block, 0, st, U, ldu, W, jrows ? 1 : R, jrows ? C : 1, Y, ldy, N, C,
+                       R, s, rpb);
     return hipGetLastError();
 }
 
@@ -891,138 +1049,162 @@ inline int colsum_splits(int N, int C) {
 }
 inline int colsum_npad(int N) { return (N + kCsRows - 1) / kCsRows * kCsRows; }
 
-// bf16: U (f32 [N, R]) -> ut (bf16, operand order) -> split partials -> out.
-template <typename TU>
-hipError_t colsum_bf16(const TU *U, int64_t ldu, const bf16 *X, int64_t ldx, float *out, int64_t os_j,
-                       int64_t os_c, int N, int C, int R, float s, bf16 *ut, float *part, hipStream_t st) {
-    const int npad = colsum_npad(N), splits = colsum_splits(N, C);
-    const int stages = npad / kCsRows;
-    const int chunk = (stages + splits - 1) / splits * kCsRows;
-    hipLaunchKernelGGL(lora_ut_kernel<TU>, dim3((unsigned)((32 * (int64_t)npad + 255) / 256)), dim3(256), 0, st, U,
-                       ldu, ut, N, R, npad);
-    hipLaunchKernelGGL(lora_colsum_mfma_kernel, dim3((unsigned)((C + kCsCols - 1) / kCsCols), (unsigned)splits),
-                       dim3(256), 0, st, X, ldx, ut, npad, part, N, C, chunk);
-    hipLaunchKernelGGL(lora_colsum_reduce_kernel, dim3((unsigned)((C * 32 + 255) / 256)), dim3(256), 0, st, part,
-                       out, os_j, os_c, C, R, splits, s);
-    return hipGetLastError();
+// Token splits of the f32 colsum: about 512 workgroups over both products
+// (`tiles` column tiles in all), a split at least 128 tokens (two blocks per
+// wave) long.
+inline int colsum_f32_splits(int N, int tiles) {
+    int sp = (512 + tiles - 1) / tiles;
+    const int most = N / 128;
+    sp = sp < most ? sp : most;
+    return sp < 1 ? 1 : sp;
 }
-
-template <typename T>
-hipError_t colsum(const float *U, int64_t ldu, const T *X, int64_t ldx, float *out, int64_t os_j,
-                  int64_t os_c, int N, int C, int R, float s, hipStream_t st) {
-    const dim3 grid((C + 63) / 64), block(256);
-    hipLaunchKernelGGL(lora_colsum_kernel<T>, grid, block, 0, st, U, ldu, X, ldx, out, os_j, os_c,
-                       N, C, R, s);
-    return hipGetLastError();
-}
-
-template <typename T>
-hipError_t transpose(const T *src, T *dst, int R, int C, hipStream_t st) {
-    const int64_t n = (int64_t)R * C;
-    hipLaunchKernelGGL(lora_transpose_kernel<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                       src, dst, R, C);
-    return hipGetLastError();
-}
-
-template <typename T>
-hipError_t lora_fwd_t(const LoraParams &p, hipStream_t st) {
-    hipError_t e = rowdot<T>(static_cast<const T *>(p.x), p.ldx, static_cast<const T *>(p.a), p.u,
-                             p.r, p.N, p.K, p.r, 1.f, st);
-    if (e != hipSuccess) return e;
-    // y += s * u B^T : B is [M, r] = Wt for expand
-    return expand<T>(p.u, p.r, static_cast<const T *>(p.b), static_cast<T *>(p.y), p.ldy, p.N, p.M,
-                     p.r, p.scale, st);
-}
+inline int colsum_f32_tiles(int K, int M) { return (K + 127) / 128 + (M + 127) / 128; }
 
 inline size_t al256(size_t x) { return (x + 255) & ~size_t(255); }
-
-// Workspace layout (bytes, each 256-aligned): du f32 [N, r] | B^T [r, M] |
-// A^T [K, r] | bf16 colsum only: ut bf16 [32, npad] | partials f32
-// [splits(N, C) * C * 32], the larger of C = K and C = M
-template <typename T>
-hipError_t lora_bwd_t(const LoraParams &p, hipStream_t st) {
-    char *ws = reinterpret_cast<char *>(p.work);
-    float *du = reinterpret_cast<float *>(ws);
-    const size_t du_b = al256((size_t)p.N * p.r * 4);
-    T *bt = reinterpret_cast<T *>(ws + du_b);
-    const size_t bt_b = al256((size_t)p.r * p.M * sizeof(T));
-    T *at = reinterpret_cast<T *>(ws + du_b + bt_b);
-    const size_t at_b = al256((size_t)p.K * p.r * sizeof(T));
-    bf16 *ut = reinterpret_cast<bf16 *>(ws + du_b + bt_b + at_b);
-    float *part = reinterpret_cast<float *>(ws + du_b + bt_b + at_b + al256((size_t)32 * colsum_npad(p.N) * 2));
-    hipError_t e;
-    // dB[o][j] = s * sum_n dy[n][o] u[n][j]
-    if constexpr (sizeof(T) == 2)
-        e = colsum_bf16<float>(p.u, p.r, static_cast<const bf16 *>(p.dy), p.lddy, p.db, 1, p.r, p.N, p.M, p.r,
-                               p.scale, ut, part, st);
-    else
-        e = colsum<T>(p.u, p.r, static_cast<const T *>(p.dy), p.lddy, p.db, 1, p.r, p.N, p.M, p.r, p.scale, st);
-    if (e != hipSuccess) return e;
-    // du = s * dy B  (B^T as the [r, M] row operand)
-    if ((e = transpose<T>(static_cast<const T *>(p.b), bt, p.M, p.r, st)) != hipSuccess) return e;
-    if ((e = rowdot<T>(static_cast<const T *>(p.dy), p.lddy, bt, du, p.r, p.N, p.M, p.r, p.scale,
-                       st)) != hipSuccess)
-        return e;
-    // dA[j][k] = sum_n du[n][j] x[n][k]
-    if constexpr (sizeof(T) == 2)
-        e = colsum_bf16<float>(du, p.r, static_cast<const bf16 *>(p.x), p.ldx, p.da, p.K, 1, p.N, p.K, p.r, 1.f,
-                               ut, part, st);
-    else
-        e = colsum<T>(du, p.r, static_cast<const T *>(p.x), p.ldx, p.da, p.K, 1, p.N, p.K, p.r, 1.f, st);
-    if (e != hipSuccess) return e;
-    if (p.dx) {
-        // dx += du A  (A^T [K, r] as Wt)
-        if ((e = transpose<T>(static_cast<const T *>(p.a), at, p.r, p.K, st)) != hipSuccess) return e;
-        if ((e = expand<T>(du, p.r, at, static_cast<T *>(p.dx), p.lddx, p.N, p.K, p.r, 1.f, st)) !=
-            hipSuccess)
-            return e;
-    }
-    return hipSuccess;
+inline int grad_rows(int R) { return R > 32 ? 64 : 32; }
+inline size_t grad_item_bytes(int N, int C, int R) {
+    return al256((size_t)grad_rows(R) * colsum_npad(N) * 2) +
+           al256((size_t)colsum_splits(N, C) * C * grad_rows(R) * 4);
 }
 
+hipError_t lora_fwd_bf16(const LoraParams &p, hipStream_t st) {
+    const hipError_t e = rowdot16<bf16, float>(static_cast<const bf16 *>(p.x), p.ldx, static_cast<const bf16 *>(p.a),
+                                               p.u, p.r, p.N, p.K, p.r, 1.f, st);
+    if (e != hipSuccess) return e;
+    // y += s * u B^T : B is [M, r] = Wt for expand
+    return expand_mfma<float>(p.u, p.r, static_cast<const bf16 *>(p.b), static_cast<bf16 *>(p.y), p.ldy, p.N, p.M, p.r,
+                              p.scale, st);
+}
+
+hipError_t lora_fwd_f32(const LoraParams &p, hipStream_t st) {
+    const hipError_t e = rowdot(static_cast<const float *>(p.x), p.ldx, static_cast<const float *>(p.a), p.u, p.r, p.N,
+                                p.K, p.r, 1.f, st);
+    if (e != hipSuccess) return e;
+    return expand_f32(p.u, p.r, static_cast<const float *>(p.b), false, static_cast<float *>(p.y), p.ldy, p.N, p.M,
+                      p.r, p.scale, st);
+}
+
+template <typename T>
+hipError_t bwd_prep(const LoraParams &p, T *bt, T *at, bf16 *ub, int ldub, hipStream_t st) {
+    BwdPrep<T> q{};
+    q.b = static_cast<const T *>(p.b);
+    q.a = static_cast<const T *>(p.a);
+    q.u = p.u;
+    q.bt = bt;
+    q.at = at;
+    q.ub = ub;
+    q.M = p.M;
+    q.K = p.K;
+    q.N = p.N;
+    q.R = p.r;
+    q.ldub = ldub;
+    auto blocks = [](int64_t n) { return (int)((n + 255) / 256); };
+    q.wg_a = blocks((int64_t)p.r * p.M);
+    q.wg_u = q.wg_a + (at ? blocks((int64_t)p.r * p.K) : 0);
+    const int total = q.wg_u + (ub ? blocks((int64_t)p.N * p.r) : 0);
+    hipLaunchKernelGGL(lora_bwd_prep_kernel<T>, dim3((unsigned)total), dim3(256), 0, st, q);
+    return hipGetLastError();
+}
+
+// f32 workspace (bytes, each 256-aligned): du f32 [N, r] | B^T [r, M] | the
+// partials of dB and dA, [splits][M or K][r] each.  Five launches: prep, du,
+// both gradients, their reduce (with one split, none), dx.
+inline size_t lora_bwd_f32_bytes(int N, int K, int M, int r) {
+    const size_t sp = (size_t)colsum_f32_splits(N, colsum_f32_tiles(K, M));
+    return al256((size_t)N * r * 4) + al256((size_t)r * M * 4) + al256(sp * M * r * 4) + al256(sp * K * r * 4);
+}
+hipError_t lora_bwd_f32(const LoraParams &p, hipStream_t st) {
+    char *ws = reinterpret_cast<char *>(p.work);
+    float *du = reinterpret_cast<float *>(ws);
+    float *bt = reinterpret_cast<float *>(ws += al256((size_t)p.N * p.r * 4));
+    hipError_t e = bwd_prep<float>(p, bt, nullptr, nullptr, 0, st);
+    if (e != hipSuccess) return e;
+    // du = s * dy B
+    const float *dy = static_cast<const float *>(p.dy), *x = static_cast<const float *>(p.x);
+    if ((e = rowdot(dy, p.lddy, bt, du, p.r, p.N, p.M, p.r, p.scale, st)) != hipSuccess) return e;
+    // dB[o][j] = s * sum_n dy[n][o] u[n][j], dA[j][k] = sum_n du[n][j] x[n][k]
+    if (p.lddy < (1 << 26) && p.ldx < (1 << 26)) {  // 16 rows within 32-bit byte offsets
+        const int sp = colsum_f32_splits(p.N, colsum_f32_tiles(p.K, p.M));
+        const int chunk = ((p.N + sp - 1) / sp + 15) / 16 * 16, splits = (p.N + chunk - 1) / chunk;
+        CsPair g{};
+        g.N = p.N;
+        g.R = p.r;
+        float *part = reinterpret_cast<float *>(ws += al256((size_t)p.r * p.M * 4));
+        g.p[0] = {p.u, p.r, dy, p.lddy, p.db, 1, p.r, part, p.scale, p.M, splits, chunk, 0};
+        part = reinterpret_cast<float *>(ws += al256((size_t)sp * p.M * p.r * 4));
+        g.p[1] = {du, p.r, x, p.ldx, p.da, p.K, 1, part, 1.f, p.K, splits, chunk, (p.M + 127) / 128 * splits};
+        const unsigned wgs = (unsigned)(g.p[1].wg0 + (p.K + 127) / 128 * splits);
+        hipLaunchKernelGGL(lora_colsum_f32_kernel, dim3(wgs), dim3(256), 0, st, g);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        if (splits > 1) {
+            const int64_t n = (int64_t)(p.K > p.M ? p.K : p.M) * p.r;
+            hipLaunchKernelGGL(lora_colsum_reduce_f32_kernel, dim3((unsigned)((n + 255) / 256), 2), dim3(256), 0, st, g);
+        }
+    } else {
+        hipLaunchKernelGGL(lora_colsum_kernel, dim3((p.M + 63) / 64), dim3(256), 0, st, p.u, p.r, dy, p.lddy, p.db, 1,
+                           p.r, p.N, p.M, p.r, p.scale);
+        hipLaunchKernelGGL(lora_colsum_kernel, dim3((p.K + 63) / 64), dim3(256), 0, st, du, p.r, x, p.ldx, p.da, p.K, 1,
+                           p.N, p.K, p.r, 1.f);
+    }
+    if ((e = hipGetLastError()) != hipSuccess || !p.dx) return e;
+    // dx += du A
+    return expand_f32(du, p.r, static_cast<const float *>(p.a), true, static_cast<float *>(p.dx), p.lddx, p.N, p.K,
+                      p.r, 1.f, st);
+}
+
+// bf16 workspace: du and u as bf16 rows of stride r rounded up to 8 | B^T [r,
+// M] | A^T [K, r] | the two gradient products' (lora_grad_many).  du is rounded
+// where it is formed: every product it enters rounds it to bf16.
+inline int bwd_ldub(int r) { return (r + 7) & ~7; }
+inline size_t lora_bwd_bf16_bytes(int N, int K, int M, int r) {
+    return 2 * al256((size_t)N * bwd_ldub(r) * 2) + al256((size_t)r * M * 2) + al256((size_t)K * r * 2) +
+           grad_item_bytes(N, M, r) + grad_item_bytes(N, K, r);
+}
 }  // namespace
 
+// Five launches: prep, du, both gradients and their reduce, dx.  Against nine
+// (a transpose, a staging of U, a product and a reduce for each gradient) the
+// forward and backward of 4096 x 3072 x 3072 at r 16 went from 98 to 67 us
+// (both gradients' products 35 -> 18 us, staging and transposes 10 -> 3, the
+// reduces 8 -> 4), same bits.
+static hipError_t lora_bwd_bf16(const LoraParams &p, hipStream_t st) {
+    char *ws = reinterpret_cast<char *>(p.work);
+    const int ld = bwd_ldub(p.r);
+    bf16 *du = reinterpret_cast<bf16 *>(ws);
+    bf16 *ub = reinterpret_cast<bf16 *>(ws += al256((size_t)p.N * ld * 2));
+    bf16 *bt = reinterpret_cast<bf16 *>(ws += al256((size_t)p.N * ld * 2));
+    bf16 *at = reinterpret_cast<bf16 *>(ws += al256((size_t)p.r * p.M * 2));
+    ws += al256((size_t)p.K * p.r * 2);
+    hipError_t e = bwd_prep<bf16>(p, bt, p.dx ? at : nullptr, ub, ld, st);
+    if (e != hipSuccess) return e;
+    // du = s * dy B  (B^T as the [r, M] row operand)
+    const bf16 *dy = static_cast<const bf16 *>(p.dy);
+    if ((e = rowdot16<bf16, bf16>(dy, p.lddy, bt, du, ld, p.N, p.M, p.r, p.scale, st)) != hipSuccess) return e;
+    // dB[o][j] = s * sum_n dy[n][o] u[n][j], dA[j][k] = sum_n du[n][j] x[n][k]
+    const LoraGradItem items[2] = {{ub, ld, p.dy, p.lddy, p.N, p.M, p.r, p.scale, p.db, true},
+                                   {du, ld, p.x, p.ldx, p.N, p.K, p.r, 1.f, p.da, false}};
+    if ((e = launch_lora_grad_many_bf16(items, 2, ws, st)) != hipSuccess || !p.dx) return e;
+    // dx += du A  (A^T [K, r] as Wt)
+    return expand_mfma<bf16>(du, ld, at, static_cast<bf16 *>(p.dx), p.lddx, p.N, p.K, p.r, 1.f, st);
+}
+
 size_t lora_bwd_workspace_bytes(int N, int K, int M, int r, int elt) {
-    const size_t base = al256((size_t)N * r * 4) + al256((size_t)r * M * elt) + al256((size_t)K * r * elt);
-    if (elt != 2) return base;
-    // the two colsum calls (C = M for dB, C = K for dA) share the partials
-    const size_t pk = (size_t)colsum_splits(N, K) * K, pm = (size_t)colsum_splits(N, M) * M;
-    return base + al256((size_t)32 * colsum_npad(N) * 2) + al256((pk > pm ? pk : pm) * 32 * 4);
+    return elt == 2 ? lora_bwd_bf16_bytes(N, K, M, r) : lora_bwd_f32_bytes(N, K, M, r);
 }
 
 hipError_t launch_lora_fwd(const LoraParams &p, int dtype, hipStream_t s) {
-    return dtype == 0 ? lora_fwd_t<bf16>(p, s) : lora_fwd_t<float>(p, s);
+    return dtype == 0 ? lora_fwd_bf16(p, s) : lora_fwd_f32(p, s);
 }
 
 hipError_t launch_lora_bwd(const LoraParams &p, int dtype, hipStream_t s) {
-    return dtype == 0 ? lora_bwd_t<bf16>(p, s) : lora_bwd_t<float>(p, s);
+    return dtype == 0 ? lora_bwd_bf16(p, s) : lora_bwd_f32(p, s);
 }
 
 // ---- bf16 pieces for adapters folded into the base GEMMs -----------------
 hipError_t launch_lora_down_bf16(const void *x, int64_t ldx, const void *a, int N, int K, int R, float scale,
                                  void *u, int64_t ldu, hipStream_t st) {
-    const bf16 *X = static_cast<const bf16 *>(x), *A = static_cast<const bf16 *>(a);
-    bf16 *U = static_cast<bf16 *>(u);
-    auto go = [&](auto mtc) {
-        constexpr int MT = decltype(mtc)::value;
-        const dim3 grid((unsigned)((N + 16 * MT - 1) / (16 * MT))), block(512);
-        // R <= 64: up to four 16-column tiles per workgroup (a stack of adapters
-        // that share x, e.g. q/k/v, runs as one product)
-        if (R <= 16)
-            hipLaunchKernelGGL((lora_rowdot16_kernel<1, bf16, MT>), grid, block, 0, st, X, ldx, A, U, ldu, N, K, R, scale);
-        else if (R <= 32)
-            hipLaunchKernelGGL((lora_rowdot16_kernel<2, bf16, MT>), grid, block, 0, st, X, ldx, A, U, ldu, N, K, R, scale);
-        else if (R <= 48)
-            hipLaunchKernelGGL((lora_rowdot16_kernel<3, bf16, MT>), grid, block, 0, st, X, ldx, A, U, ldu, N, K, R, scale);
-        else
-            hipLaunchKernelGGL((lora_rowdot16_kernel<4, bf16, MT>), grid, block, 0, st, X, ldx, A, U, ldu, N, K, R, scale);
-    };
-    switch (rowdot_slabs(N, (R + 15) / 16)) {
-    case 1: go(std::integral_constant<int, 1>{}); break;
-    case 2: go(std::integral_constant<int, 2>{}); break;
-    default: go(std::integral_constant<int, 4>{}); break;
-    }
-    return hipGetLastError();
+    return rowdot16<bf16, bf16>(static_cast<const bf16 *>(x), ldx, static_cast<const bf16 *>(a), static_cast<bf16 *>(u),
+                                ldu, N, K, R, scale, st);
 }
 
 hipError_t launch_lora_up_bf16(const void *u, int64_t ldu, const void *b, int N, int M, int R, float scale, void *y,
@@ -1030,14 +1212,6 @@ hipError_t launch_lora_up_bf16(const void *u, int64_t ldu, const void *b, int N,
     return expand_mfma<bf16>(static_cast<const bf16 *>(u), ldu, static_cast<const bf16 *>(b), static_cast<bf16 *>(y),
                              ldy, N, M, R, scale, st);
 }
-
-namespace {
-inline int grad_rows(int R) { return R > 32 ? 64 : 32; }
-inline size_t grad_item_bytes(int N, int C, int R) {
-    return al256((size_t)grad_rows(R) * colsum_npad(N) * 2) +
-           al256((size_t)colsum_splits(N, C) * C * grad_rows(R) * 4);
-}
-}  // namespace
 
 size_t lora_grad_many_workspace_bytes(const LoraGradItem *items, int count) {
     // sets of kGradMany products run one after another over the same bytes
