@@ -20,7 +20,8 @@
 //   3. dq:     one workgroup per NW*32 queries (NW waves x 32), looping over
 //              32-key LDS units.  S^T = K Q^T puts queries on the lanes, so
 //              dS^T feeds dQ^T = K^T dS^T as the B operand.
-// With a workspace for it (8-wave bf16 grids, p.ds), dK/dV also stores every
+// With 4-wave workgroups 2 and 3 run as one grid (attn_bwd_pair_bf16_kernel).
+// With a workspace for it (8-wave D = 128 grids, p.ds), dK/dV also stores every
 // bf16 dS value and dQ becomes 3': an HBM-bound dQ^T = K^T dS^T over the
 // stored dS, the same products in the same key order as 3, so the same bits
 // without 3's recompute of S and dP (2 of its 3G of matrix work).
@@ -44,6 +45,15 @@ namespace {
 // written once and read once; measured 2-4% off the backward at c2 and c5
 // against the default policy).
 constexpr int kDsCachePolicy = 2;
+
+// LDS object I of BYTES bytes.  Stage buffers are distinct objects, so that the
+// compiler keeps the prefetch DMA into one in flight across reads of another.
+// Two blocks that name the same object share it in a kernel holding both.
+template <int I, int BYTES>
+__device__ __forceinline__ char *lds_obj() {
+    __shared__ __align__(16) char x[BYTES];
+    return x;
+}
 
 // ---------------------------------------------------------------------------
 // 1. delta = rowsum(dO * O) in f32, written [B,H,S]; also lse2 = LSE*log2(e)
@@ -101,11 +111,6 @@ template <int D, int NW>
 struct DkvTile {
     using T = LdsTile<D, kQB>;
     static constexpr int KT = NW * 32;  // keys per workgroup
-    static constexpr int Q_OFF = 0;
-    static constexpr int DO_OFF = T::BYTES;
-    static constexpr int LSE_OFF = 2 * T::BYTES;        // 64 f32
-    static constexpr int DELTA_OFF = LSE_OFF + kQB * 4;  // 64 f32
-    static constexpr int STAGE = DELTA_OFF + kQB * 4;
     static constexpr int WI = T::WAVE_INSTS / NW;
     static_assert(WI >= 1 && WI * NW == T::WAVE_INSTS, "tile split over waves");
 };
@@ -119,7 +124,10 @@ struct DkvTile {
 // [key / 32][q / 16] with ds_ld / 16 blocks per row.  One permlane32 swap per
 // word puts 8 consecutive queries of the lane's key in each lane, so a wave
 // stores a whole block with one 16-byte store per lane.
-template <int D, int NW, bool SPLIT, bool DS = false>
+// PAIR: the stage tiles are the dQ block's buffers (objects 0 .. 3) and their
+// row vectors objects of their own; otherwise a stage is one object (with four
+// tile objects the 256-register kernels spill two more).
+template <int D, int NW, bool SPLIT, bool DS = false, bool PAIR = false>
 __device__ __forceinline__ void dkdv_block(const AttnBwdParams &p, int work) {
     static_assert(!(SPLIT && DS), "dS is stored by the unsplit kernel only");
     using F = DkvTile<D, NW>;
@@ -185,21 +193,24 @@ __device__ __forceinline__ void dkdv_block(const AttnBwdParams &p, int work) {
     const uint32_t ovo = tile_src_off<D>(wave, lane, p.do_ss);
     const uint32_t qi_step = tile_inst_row_step<D, NW>(p.q_ss), oi_step = tile_inst_row_step<D, NW>(p.do_ss);
     const uint32_t qstep = (uint32_t)(kQB * p.q_ss * 2), ostep = (uint32_t)(kQB * p.do_ss * 2);
-    // one LDS object per stage: the compiler then keeps the prefetch DMA in
-    // flight across the transpose reads of the other stage
-    __shared__ __align__(16) char stage0[F::STAGE], stage1[F::STAGE];
+    // per stage: a Q tile, a dO tile, and 64 lse2 then 64 delta values
+    constexpr int ROWV = 2 * kQB * 4;
+    char *const qst[2] = {PAIR ? lds_obj<0, T::BYTES>() : lds_obj<4, 2 * T::BYTES + ROWV>(),
+                          PAIR ? lds_obj<2, T::BYTES>() : lds_obj<5, 2 * T::BYTES + ROWV>()};
+    char *const ost[2] = {PAIR ? lds_obj<1, T::BYTES>() : qst[0] + T::BYTES,
+                          PAIR ? lds_obj<3, T::BYTES>() : qst[1] + T::BYTES};
+    char *const rst[2] = {PAIR ? lds_obj<6, ROWV>() : ost[0] + T::BYTES, PAIR ? lds_obj<7, ROWV>() : ost[1] + T::BYTES};
     auto issue = [&](int qb, int buf) {
-        char *st = buf ? stage1 : stage0;
 #pragma unroll
         for (int i = 0; i < F::WI; ++i)
-            buffer_to_lds_16(qrs, st + F::Q_OFF + (i * NW + wave) * 1024, qvo, qb * qstep + i * qi_step);
+            buffer_to_lds_16(qrs, qst[buf] + (i * NW + wave) * 1024, qvo, qb * qstep + i * qi_step);
 #pragma unroll
         for (int i = 0; i < F::WI; ++i)
-            buffer_to_lds_16(ors, st + F::DO_OFF + (i * NW + wave) * 1024, ovo, qb * ostep + i * oi_step);
+            buffer_to_lds_16(ors, ost[buf] + (i * NW + wave) * 1024, ovo, qb * ostep + i * oi_step);
         if (wave == 0)
-            buffer_to_lds_4(lrs, st + F::LSE_OFF, lane * 4, qb * kQB * 4);
+            buffer_to_lds_4(lrs, rst[buf], lane * 4, qb * kQB * 4);
         else if (wave == 1)
-            buffer_to_lds_4(drs, st + F::DELTA_OFF, lane * 4, qb * kQB * 4);
+            buffer_to_lds_4(drs, rst[buf] + kQB * 4, lane * 4, qb * kQB * 4);
     };
 
     // loop-invariant LDS operand offsets
@@ -247,10 +258,9 @@ __device__ __forceinline__ void dkdv_block(const AttnBwdParams &p, int work) {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (qb + 1 < qb1) issue(qb + 1, P ^ 1);
-        const char *st = P ? stage1 : stage0;
-        const char *qs_t = st + F::Q_OFF, *os_t = st + F::DO_OFF;
-        const float *lse_s = reinterpret_cast<const float *>(st + F::LSE_OFF);
-        const float *dlt_s = reinterpret_cast<const float *>(st + F::DELTA_OFF);
+        const char *qs_t = qst[P], *os_t = ost[P];
+        const float *lse_s = reinterpret_cast<const float *>(rst[P]);
+        const float *dlt_s = lse_s + kQB;
 
 #pragma unroll 1
         for (int sub = 0; sub < kQB / 32; ++sub) {
@@ -435,10 +445,12 @@ __device__ __forceinline__ void dq_block(const AttnBwdParams &p, int work) {
     const __amdgpu_buffer_rsrc_t keep_rs = make_rsrc(keep, (uint32_t)S);
     if (track) live_mask_issue<NW, 4 * kKU, kLiveU>(keep_rs, u0 >> 2, live, lv);
 
-    // distinct LDS objects per buffer (see attn_fwd.hip: lets the compiler
-    // keep the prefetch DMA in flight across reads of the other buffers)
-    __shared__ __align__(16) char k0[T::BYTES], k1[T::BYTES], k2[T::BYTES], k3[T::BYTES];
-    __shared__ __align__(16) char v0[T::BYTES], v1[T::BYTES], v2[T::BYTES], v3[T::BYTES];
+    // one LDS object per buffer, its K unit then its V unit: a unit reads
+    // buffers i and i + 1 while the DMA fills i + 3
+    char *const k0 = lds_obj<0, 2 * T::BYTES>(), *const v0 = k0 + T::BYTES;
+    char *const k1 = lds_obj<1, 2 * T::BYTES>(), *const v1 = k1 + T::BYTES;
+    char *const k2 = lds_obj<2, 2 * T::BYTES>(), *const v2 = k2 + T::BYTES;
+    char *const k3 = lds_obj<3, 2 * T::BYTES>(), *const v3 = k3 + T::BYTES;
     auto kb_ = [&](int i) -> char * { return i == 0 ? k0 : i == 1 ? k1 : i == 2 ? k2 : k3; };
     auto vb_ = [&](int i) -> char * { return i == 0 ? v0 : i == 1 ? v1 : i == 2 ? v2 : v3; };
 
@@ -822,6 +834,18 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_bwd_dq_bf16_kernel(AttnBwdPar
     dq_block<D, KEEP, NW, DELTA, SPLIT>(p, xcd_remap(blockIdx.x, gridDim.x));
 }
 
+// dK/dV and dQ of 4-wave shapes in one grid, after the pre-pass: the longer
+// dK/dV workgroups first, dQ's fill the CUs they leave.  (They are independent
+// after the pre-pass; 8-wave workgroups each fill a CU and stay separate.)
+template <int D, bool KEEP>
+__global__ __launch_bounds__(256, 2) void attn_bwd_pair_bf16_kernel(AttnBwdParams p, int n_dkdv) {
+    const int b = blockIdx.x;
+    if (b < n_dkdv)
+        dkdv_block<D, 4, false, false, true>(p, xcd_remap(b, n_dkdv));
+    else
+        dq_block<D, KEEP, 4, false, false>(p, xcd_remap(b - n_dkdv, (int)gridDim.x - n_dkdv));
+}
+
 template <int D, int NW, bool DELTA, bool SPLIT>
 void launch_dq(const AttnBwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
     if (p.keep)
@@ -921,79 +945,78 @@ hipError_t launch_attn_bwd_split(const AttnBwdParams &p, int D, int phase, hipSt
     return phase == 0 ? launch_reduce(p, D, 0, 3, s) : launch_reduce(p, D, 1, 2, s);
 }
 
-// Unsplit backward through the stored dS^T (p.ds): pre-pass, dK/dV storing
-// dS^T, then dQ from it -- in this order (dQ reads what dK/dV stored).
-hipError_t launch_attn_bwd_ds(const AttnBwdParams &p, int D, int phase, hipStream_t s) {
+// Unsplit D = 128 backward through the stored dS^T (p.ds, 8-wave grids):
+// pre-pass, dK/dV storing dS^T, then dQ from it -- in this order (dQ reads
+// what dK/dV stored).
+hipError_t launch_attn_bwd_ds(const AttnBwdParams &p, int phase, hipStream_t s) {
     hipError_t e = hipSuccess;
+    const dim3 grid(p.B * p.H * ((p.S + 255) / 256)), block(512);
     if (phase == 0 || phase == 1) {
-        e = D == 128 ? launch_delta<bf16, 128>(p, s) : launch_delta<bf16, 64>(p, s);
-        if (e != hipSuccess) return e;
+        if ((e = launch_delta<bf16, 128>(p, s)) != hipSuccess) return e;
     }
     if (phase == 0 || phase == 2) {
-        const int nw = attn_waves(p.B, p.H, p.S);
-        const dim3 grid(p.B * p.H * ((p.S + nw * 32 - 1) / (nw * 32))), block(nw * 64);
-        if (D == 128 && nw == 8)
-            hipLaunchKernelGGL((attn_bwd_dkdv_bf16_kernel<128, 8, false, true>), grid, block, 0, s, p);
-        else if (D == 128)
-            hipLaunchKernelGGL((attn_bwd_dkdv_bf16_kernel<128, 4, false, true>), grid, block, 0, s, p);
-        else if (nw == 8)
-            hipLaunchKernelGGL((attn_bwd_dkdv_bf16_kernel<64, 8, false, true>), grid, block, 0, s, p);
-        else
-            hipLaunchKernelGGL((attn_bwd_dkdv_bf16_kernel<64, 4, false, true>), grid, block, 0, s, p);
+        hipLaunchKernelGGL((attn_bwd_dkdv_bf16_kernel<128, 8, false, true>), grid, block, 0, s, p);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (phase == 0 || phase == 3) {
-        const dim3 grid(p.B * p.H * ((p.S + DqDsTile<128>::QT - 1) / DqDsTile<128>::QT)), block(512);
-        if (D == 128)
-            hipLaunchKernelGGL(attn_bwd_dq_ds_kernel<128>, grid, block, 0, s, p);
-        else
-            hipLaunchKernelGGL(attn_bwd_dq_ds_kernel<64>, grid, block, 0, s, p);
+        hipLaunchKernelGGL(attn_bwd_dq_ds_kernel<128>, grid, block, 0, s, p);
         e = hipGetLastError();
     }
     return e;
 }
 
+// Workgroup shape as for the forward (attn_waves) at D = 128.  At D = 64 4
+// waves throughout: the kernels' registers let three waves share a SIMD, and
+// dK/dV and dQ run in one grid (B1 H24 S4608 D64 562 -> 471 us, B4 S1536 281
+// -> 213, B1 S1536 88 -> 70).
 hipError_t launch_attn_bwd_bf16(const AttnBwdParams &p, int D, int phase, hipStream_t s) {
     if (p.split > 1) return launch_attn_bwd_split(p, D, phase, s);
-    if (p.ds) return launch_attn_bwd_ds(p, D, phase, s);
-    // workgroup shape as for the forward (attn_waves); dQ at D = 64 streams
-    // 4 KiB units, too small to split over 8 waves.
-    const int nw = attn_waves(p.B, p.H, p.S);
-    const int nw_q = D == 128 ? nw : 4;
-    // The whole backward with 8-wave kernels runs in order on one stream:
-    // dQ first, doing the pre-pass for its own queries, then dK/dV.
-    const bool fused = phase == 0 && nw == 8;
+    if (p.ds) return launch_attn_bwd_ds(p, phase, s);
+    const int nw = D == 128 ? attn_waves(p.B, p.H, p.S) : 4;
+    const int n = p.B * p.H * ((p.S + nw * 32 - 1) / (nw * 32));  // workgroups of each kernel
+    const dim3 grid(n), block(nw * 64);
+    // The whole backward in two launches: with 8-wave kernels dQ first, doing
+    // the pre-pass for its own queries, then dK/dV; with 4-wave kernels the
+    // pre-pass, then dK/dV and dQ in one grid.  (Against dQ on a second stream
+    // beside dK/dV, joined by events, the one grid saves 45 us of host time a
+    // call, and on the GPU B2 H24 S333 49 -> 32 us, B4 H24 S1536 409 -> 406.)
+    const bool fused = phase == 0 && nw == 8, pair = phase == 0 && nw == 4;
     hipError_t e = hipSuccess;
-    if (!fused && (phase == 0 || phase == 1)) {
+    if (pair || phase == 1) {
         e = D == 128 ? launch_delta<bf16, 128>(p, s) : launch_delta<bf16, 64>(p, s);
         if (e != hipSuccess) return e;
     }
-    auto dq = [&](bool delta) {
-        const dim3 grid(p.B * p.H * ((p.S + nw_q * 32 - 1) / (nw_q * 32))), block(nw_q * 64);
-        if (D == 128 && nw_q == 8)
-            delta ? launch_dq<128, 8, true, false>(p, grid, block, s)
+    if (pair) {
+        const dim3 pgrid(2 * n);
+        if (D == 128 && p.keep)
+            hipLaunchKernelGGL((attn_bwd_pair_bf16_kernel<128, true>), pgrid, block, 0, s, p, n);
+        else if (D == 128)
+            hipLaunchKernelGGL((attn_bwd_pair_bf16_kernel<128, false>), pgrid, block, 0, s, p, n);
+        else if (p.keep)
+            hipLaunchKernelGGL((attn_bwd_pair_bf16_kernel<64, true>), pgrid, block, 0, s, p, n);
+        else
+            hipLaunchKernelGGL((attn_bwd_pair_bf16_kernel<64, false>), pgrid, block, 0, s, p, n);
+        return hipGetLastError();
+    }
+    if (fused || phase == 3) {
+        if (nw == 8)
+            fused ? launch_dq<128, 8, true, false>(p, grid, block, s)
                   : launch_dq<128, 8, false, false>(p, grid, block, s);
         else if (D == 128)
-            delta ? launch_dq<128, 4, true, false>(p, grid, block, s)
-                  : launch_dq<128, 4, false, false>(p, grid, block, s);
+            launch_dq<128, 4, false, false>(p, grid, block, s);
         else
-            delta ? launch_dq<64, 4, true, false>(p, grid, block, s) : launch_dq<64, 4, false, false>(p, grid, block, s);
-        return hipGetLastError();
-    };
-    if (fused && (e = dq(true)) != hipSuccess) return e;
-    if (phase == 0 || phase == 2) {
-        const dim3 grid(p.B * p.H * ((p.S + nw * 32 - 1) / (nw * 32))), block(nw * 64);
-        if (D == 128 && nw == 8)
+            launch_dq<64, 4, false, false>(p, grid, block, s);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+    if (fused || phase == 2) {
+        if (nw == 8)
             hipLaunchKernelGGL((attn_bwd_dkdv_bf16_kernel<128, 8, false>), grid, block, 0, s, p);
         else if (D == 128)
             hipLaunchKernelGGL((attn_bwd_dkdv_bf16_kernel<128, 4, false>), grid, block, 0, s, p);
-        else if (nw == 8)
-            hipLaunchKernelGGL((attn_bwd_dkdv_bf16_kernel<64, 8, false>), grid, block, 0, s, p);
         else
             hipLaunchKernelGGL((attn_bwd_dkdv_bf16_kernel<64, 4, false>), grid, block, 0, s, p);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+        e = hipGetLastError();
     }
-    if (!fused && (phase == 0 || phase == 3)) e = dq(false);
     return e;
 }
 

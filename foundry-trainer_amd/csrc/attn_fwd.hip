@@ -487,13 +487,6 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(AttnFwdParams p) 
 
 }  // namespace
 
-// Workgroup shape, shared by the forward and backward bf16 kernels.  An
-// 8-wave workgroup fills a CU's registers alone (2 waves per SIMD), so its
-// grid runs in whole-CU rounds; 4-wave workgroups pair up per CU, and in a
-// sparse last round run alone at higher speed.  8 waves halve the streamed
-// L2 -> LDS bytes per FLOP but only pay when the 8-wave grid's last round is
-// at least half full: measured on MI355X, c2 (B1 H24 S4608: last round 69%
-// full) +3.6% and c5 (B2 S6656: 88%) +3% fwd+bwd, c3 (B4 S1536: 25%) -13%.
 // CU count of the current device (cached per device; 256 if unknown).
 int device_cu_count() {
     static int cus[64];
@@ -509,9 +502,19 @@ int device_cu_count() {
     return n;
 }
 
+// Workgroup shape of the unsplit bf16 kernels (the backward's at D = 128; at D
+// = 64 it takes 4 waves throughout, see launch_attn_bwd_bf16).  An
+// 8-wave workgroup fills a CU's registers alone (2 waves per SIMD), so its
+// grid runs in whole-CU rounds; 4-wave workgroups pair up per CU, and in a
+// sparse last round run alone at higher speed.  8 waves halve the streamed
+// L2 -> LDS bytes per FLOP but only pay when the 8-wave grid's last round is
+// at least half full: measured on MI355X, c2 (B1 H24 S4608: last round 69%
+// full) +3.6% and c5 (B2 S6656: 88%) +3% fwd+bwd, c3 (B4 S1536: 25%) -13%.
+// Grids too small for a round (those attn_split names) take 4 waves, one
+// workgroup to a CU: B1 H3 S4608 forward 107 -> 70 us, backward 343 -> 207.
 int attn_waves(int B, int H, int S) {
     if (S < 512) return 4;  // fewer than two 256-row tiles per (b, h)
-    if (attn_split(B, H, S) > 1) return 8;
+    if (attn_split(B, H, S) > 1) return 4;
     const int n = device_cu_count();
     const int64_t wg = (int64_t)B * H * ((S + 255) / 256);
     const int64_t last = wg % n == 0 ? n : wg % n;
@@ -535,6 +538,16 @@ int attn_split(int B, int H, int S) {
     split = split < 16 ? split : 16;
     return split > 1 ? (int)split : 1;
 }
+
+// Whether a split of a grid's ranges beats running it unsplit with one 4-wave
+// workgroup per CU.  The split's extra launch, partials and 8-wave ranges cost
+// about 15 us forward and 30 us backward; half a chain saved repays that only
+// from S = 4608 on, two thirds or more from the shortest sequences that split
+// so far.  Forward + backward us, split against unsplit, D = 128: in two B1 H24
+// S1024 124 / 92, H10 S3072 243 / 229, H6 S4608 309 / 311, H4 S6656 406 / 428;
+// in three H6 S1536 106 / 103, H3 S1700 107 / 112, H7 S3072 189 / 198; in four
+// H4 S2048 106 / 128, H3 S4608 186 / 278.
+bool attn_split_pays(int S, int split) { return split > 2 || (split == 2 && S >= 4608); }
 
 size_t attn_split_elems(int B, int H, int S, int D, int split) {
     return split > 1 ? (size_t)split * B * H * S * D : 0;

@@ -174,9 +174,14 @@ fa_status check_buffer_view(const char *name, const fa_strides &st, int32_t S, i
 
 size_t round256(size_t x) { return (x + 255) & ~size_t(255); }
 
-// Range split factor of a bf16 call (1 for f32 or unsplit shapes).
+// Range split factor the workspaces hold room for (1 for f32 or shapes that
+// never split), and the one a call runs with.
 int split_for(int32_t dtype, int32_t B, int32_t S, int32_t H) {
     return dtype == FA_DTYPE_BF16 ? fa::attn_split(B, H, S) : 1;
+}
+int split_used(int32_t dtype, int32_t B, int32_t S, int32_t H) {
+    const int split = split_for(dtype, B, S, H);
+    return fa::attn_split_pays(S, split) ? split : 1;
 }
 
 // backward workspace: delta [B,H,S] f32, lse2 [B,H,S] f32, then for a split
@@ -213,14 +218,20 @@ size_t bwd_ds_bytes(int32_t dtype, int32_t B, int32_t S, int32_t H) {
     return bytes > (size_t)FA_BWD_DS_MAX_BYTES ? 0 : bytes;
 }
 
+// bf16 dS pays at D = 128 only: at D = 64 its traffic is the same for half the
+// products saved, and the 4-wave recomputing kernels are faster (B1 H24 S4608
+// D64: 562 us through dS, 471 recomputing).
+bool stores_ds(int32_t dtype, int32_t D) { return dtype == FA_DTYPE_F32 || D == 128; }
+
 size_t bwd_ds_workspace(int32_t dtype, int32_t B, int32_t S, int32_t H, int32_t D) {
-    return bwd_min_workspace(dtype, B, S, H, D) + bwd_ds_bytes(dtype, B, S, H);
+    return bwd_min_workspace(dtype, B, S, H, D) + (stores_ds(dtype, D) ? bwd_ds_bytes(dtype, B, S, H) : 0);
 }
 
 // What a caller that asks no further is told: f32 calls keep their rows only
-// (their dS is twice bf16's size), bf16 ones get their dS where it pays.
+// (their dS is twice bf16's size), bf16 ones get room for dS, at D = 64 too
+// (a size callers may have fixed; those calls leave it unused).
 size_t bwd_workspace(int32_t dtype, int32_t B, int32_t S, int32_t H, int32_t D) {
-    return dtype == FA_DTYPE_F32 ? bwd_min_workspace(dtype, B, S, H, D) : bwd_ds_workspace(dtype, B, S, H, D);
+    return bwd_min_workspace(dtype, B, S, H, D) + (dtype == FA_DTYPE_F32 ? 0 : bwd_ds_bytes(dtype, B, S, H));
 }
 
 // forward workspace of a split call: O partials [split][B,H,S][D] f32, then
@@ -299,7 +310,7 @@ fa_status fa_attn_fwd(const fa_attn_fwd_args *a, void *stream) {
                         "workspace of %zu bytes is smaller than the %zu a split forward needs (NULL runs unsplit)",
                         a->workspace_bytes, need);
         if (need > 0) {
-            p.split = split_for(a->dtype, a->batch, a->seq, a->heads);
+            p.split = split_used(a->dtype, a->batch, a->seq, a->heads);
             p.part_o = static_cast<float *>(a->workspace);
             p.part_lse = reinterpret_cast<float *>(
                 static_cast<char *>(a->workspace) +
@@ -340,71 +351,6 @@ fa_status fa_attn_bwd(const fa_attn_bwd_args *a, void *stream) {
 }  // extern "C"
 
 namespace {
-// With the 4-wave kernels (fa::attn_waves) the whole bf16 backward runs dQ beside
-// dK/dV: the two kernels are independent after the pre-pass, and two
-// 4-wave workgroups per CU let them fill the partial last wave each leaves
-// on its own (measured 2.4% off a 4-wave c2 backward, results
-// bit-identical).  The 8-wave kernels each fill a CU's registers alone, and
-// there running them side by side measured 4% slower than in order, so they
-// run in order on the caller's stream.  Per host thread and device: one side
-// stream (default priority) and two events, made on first use and kept for
-// the thread's life, so concurrent callers on other threads never share
-// them.
-struct BwdFork {
-    hipStream_t side = nullptr;
-    hipEvent_t pre = nullptr, done = nullptr;
-};
-constexpr int kMaxForkDevices = 64;
-thread_local BwdFork g_fork[kMaxForkDevices];
-
-hipError_t fork_for_current(BwdFork **out) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    if (dev < 0 || dev >= kMaxForkDevices) return hipErrorInvalidDevice;
-    BwdFork &f = g_fork[dev];
-    if (!f.side) {
-        hipStream_t st = nullptr;
-        hipEvent_t e0 = nullptr, e1 = nullptr;
-        // a partial failure releases what was made (the caller then runs the
-        // backward in order on its own stream)
-        if ((e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking)) != hipSuccess) return e;
-        if ((e = hipEventCreateWithFlags(&e0, hipEventDisableTiming)) != hipSuccess) {
-            (void)hipStreamDestroy(st);
-            return e;
-        }
-        if ((e = hipEventCreateWithFlags(&e1, hipEventDisableTiming)) != hipSuccess) {
-            (void)hipEventDestroy(e0);
-            (void)hipStreamDestroy(st);
-            return e;
-        }
-        f.side = st;
-        f.pre = e0;
-        f.done = e1;
-    }
-    *out = &f;
-    return hipSuccess;
-}
-
-// pre-pass and dK/dV on s; dQ on the side stream after the pre-pass; s then
-// waits for dQ, so everything the caller queues on s afterwards sees all
-// three results (and may reuse the workspace).
-hipError_t launch_bwd_forked(const fa::AttnBwdParams &p, int D, hipStream_t s) {
-    // through the stored dS, dQ follows dK/dV
-    if (p.ds || fa::attn_waves(p.B, p.H, p.S) == 8) return fa::launch_attn_bwd_bf16(p, D, FA_BWD_ALL, s);
-    BwdFork *f = nullptr;
-    if (fork_for_current(&f) != hipSuccess) return fa::launch_attn_bwd_bf16(p, D, FA_BWD_ALL, s);
-    hipError_t e = fa::launch_attn_bwd_bf16(p, D, FA_BWD_PREPASS, s);
-    if (e == hipSuccess) e = hipEventRecord(f->pre, s);
-    if (e == hipSuccess) e = fa::launch_attn_bwd_bf16(p, D, FA_BWD_DKDV, s);
-    if (e == hipSuccess) e = hipStreamWaitEvent(f->side, f->pre, 0);
-    if (e == hipSuccess) e = fa::launch_attn_bwd_bf16(p, D, FA_BWD_DQ, f->side);
-    if (e == hipSuccess) e = hipEventRecord(f->done, f->side);
-    if (e == hipSuccess) e = hipStreamWaitEvent(s, f->done, 0);
-    return e;
-}
-
-
 // Validates a backward call's shapes, views and LSE (not its workspace).
 fa_status check_bwd_args(const fa_attn_bwd_args *a) {
     FA_TRY(check_attn_shape(a->dtype, a->batch, a->seq, a->heads, a->head_dim, a->scale));
@@ -480,11 +426,10 @@ fa_status fa_attn_bwd_phase(const fa_attn_bwd_args *a, int32_t phase, void *stre
     FA_TRY(init_current());
 
     fa::AttnBwdParams p;
-    fill_bwd_params(a, static_cast<char *>(a->workspace), split_for(a->dtype, a->batch, a->seq, a->heads),
-                    ds > 0 && a->workspace_bytes >= need + ds, p);
+    fill_bwd_params(a, static_cast<char *>(a->workspace), split_used(a->dtype, a->batch, a->seq, a->heads),
+                    ds > 0 && a->workspace_bytes >= need + ds && stores_ds(a->dtype, a->head_dim), p);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const hipError_t e = a->dtype != FA_DTYPE_BF16 ? fa::launch_attn_bwd_f32(p, a->head_dim, phase, s)
-                         : phase == FA_BWD_ALL     ? launch_bwd_forked(p, a->head_dim, s)
                                                    : fa::launch_attn_bwd_bf16(p, a->head_dim, phase, s);
     if (e != hipSuccess) return hip_fail(e, "attention backward launch");
     return ok();
@@ -506,8 +451,7 @@ fa_status fa_attn_bwd_noalloc(const fa_attn_bwd_args *a, void *stream) {
     char *ws = nullptr;
     FA_TRY(scratch_for_current(&ws));
 
-    // never split (the split partials would not fit), every launch in order on
-    // the caller's stream (no side stream to create)
+    // never split: the split partials would not fit
     fa::AttnBwdParams p;
     fill_bwd_params(a, ws, 1, false, p);
     hipStream_t s = static_cast<hipStream_t>(stream);

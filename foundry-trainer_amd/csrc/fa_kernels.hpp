@@ -62,13 +62,15 @@ hipError_t launch_attn_fwd_f32(const AttnFwdParams &p, int D, hipStream_t s);
 // phase: 0 all, 1 pre-pass, 2 dK/dV, 3 dQ
 hipError_t launch_attn_bwd_bf16(const AttnBwdParams &p, int D, int phase, hipStream_t s);
 // Waves per workgroup (4 or 8, i.e. 128- or 256-row tiles) of the bf16
-// forward, dK/dV and D = 128 dQ kernels for B x H sequences of S tokens on
-// the current device (see attn_fwd.hip).
+// forward and the D = 128 backward kernels for B x H sequences of S tokens on
+// the current device (see attn_fwd.hip), when they run unsplit.
 int attn_waves(int B, int H, int S);
 // Range split factor (1 = none) of the bf16 kernels for B x H sequences of S
 // tokens on the current device: > 1 when even 8-wave workgroups would leave
 // most CUs idle (e.g. one GPU's share of heads under sequence parallelism).
 int attn_split(int B, int H, int S);
+// Whether such a split of S rows is faster than the unsplit kernels.
+bool attn_split_pays(int S, int split);
 // f32 elements of the split partials per gradient or O (split * B*H*S*D).
 size_t attn_split_elems(int B, int H, int S, int D, int split);
 hipError_t launch_attn_bwd_f32(const AttnBwdParams &p, int D, int phase, hipStream_t s);

@@ -87,7 +87,7 @@ def attn_fwd(q, k, v, scale: Optional[float] = None, key_keep=None, out=None, ls
     to 1/sqrt(D) (the reference hard-codes 1/sqrt(128), lib.rs:138).
     key_keep: optional (B,S) bool/uint8 mask, False = key excluded.
     split: pass a workspace so that a grid too small for the GPU (few heads,
-    fa_attn_fwd_workspace_size > 0) splits each tile's keys; `workspace` is
+    fa_attn_fwd_workspace_size > 0) may split each tile's keys; `workspace` is
     used when large enough, else one is allocated.  split=False runs the
     unsplit kernel.
     Returns o (same shape as q) and lse (B,H,S) float32.
@@ -128,8 +128,10 @@ def attn_bwd_workspace_bytes(B: int, S: int, H: int, D: int, dtype=torch.bfloat1
     or, with minimum, the least fa_attn_bwd accepts (dQ recomputes S and dP).
     Both give the same bits."""
     ba = _abi.AttnBwdArgs(dtype=_dtype_code(torch.empty(0, dtype=dtype)), batch=B, seq=S, heads=H, head_dim=D)
-    f = lib().fa_attn_bwd_min_workspace_size if minimum else lib().fa_attn_bwd_ds_workspace_size
-    return int(f(ctypes.byref(ba)))
+    if minimum:
+        return int(lib().fa_attn_bwd_min_workspace_size(ctypes.byref(ba)))
+    return int(max(lib().fa_attn_bwd_workspace_size(ctypes.byref(ba)),
+                   lib().fa_attn_bwd_ds_workspace_size(ctypes.byref(ba))))
 
 
 def attn_workspace_bytes(q) -> Tuple[int, int]:

@@ -104,16 +104,17 @@ typedef struct fa_attn_fwd_args {
  * when B x H x ceil(S/256) workgroups would leave at least half of the
  * current device's CUs idle and S >= 1024 (for example 3 or 6 heads at
  * S = 4608: one GPU's share of 24 heads over 8 or 4 GPUs).  Each query tile's
- * keys are then cut into up to 16 ranges of >= 512 keys on separate
- * workgroups, whose f32 partials are merged through their LSEs.  0 means
- * the forward never splits these shapes.  No reference counterpart. */
+ * keys may then be cut into up to 16 ranges of >= 512 keys on separate
+ * workgroups, whose f32 partials are merged through their LSEs (where that is
+ * faster: three ranges or more, or two from seq 4608 on).  0 means the forward
+ * never splits these shapes.  No reference counterpart. */
 size_t fa_attn_fwd_workspace_size(const fa_attn_fwd_args *args);
 
 /* O = softmax(Q K^T * scale) V per (b, h), scores and softmax in f32, P cast to
  * the storage dtype before P V (lib.rs:131-149), plus the per-row LSE that the
  * backward uses to recompute P.  A fully masked row gives O = 0, LSE = -inf.
  * With workspace NULL the call never splits; with a workspace of at least
- * fa_attn_fwd_workspace_size bytes it splits the shapes that size covers (a
+ * fa_attn_fwd_workspace_size bytes it may split the shapes that size covers (a
  * smaller non-NULL workspace is FA_ERR_INVALID_ARG).  Results are
  * deterministic either way.  Replaces AttnBwd::cuda_fwd (lib.rs:189-214) and
  * AttnBwd::cpu_fwd (lib.rs:158-187). */
@@ -168,16 +169,15 @@ size_t fa_attn_bwd_ds_workspace_size(const fa_attn_bwd_args *args);
 
 /* dQ, dK, dV of the forward above: P is recomputed from Q, K and the saved
  * LSE; dS = P * (dP - rowsum(dO * O)) * scale; dQ = dS K, dK = dS^T Q,
- * dV = P^T dO, f32 accumulation, deterministic (no atomics).  For bf16 with
- * 4-wave (128-row) workgroups -- seq < 512, or an 8-wave grid whose last
- * round would be under half full -- the dQ kernel runs on a library-owned
- * side stream (one per host thread and device, default priority) beside
- * dK/dV, joined back to `stream` by events before the call returns.  With
- * 8-wave workgroups the launches run in order on `stream`: with the full
+ * dV = P^T dO, f32 accumulation, deterministic (no atomics).  All launches run
+ * in order on `stream`.  For bf16 with 4-wave (128-row) workgroups -- seq <
+ * 512, head_dim 64, grids too small for the GPU, or an 8-wave grid whose last
+ * round would be under half full -- they are the pre-pass, then dK/dV and dQ
+ * (recomputing S and dP) in one grid.  With 8-wave workgroups: with the full
  * workspace the pre-pass, dK/dV (also storing dS), then dQ = dS K * scale
  * read from the stored dS; with the minimum one dQ (which also forms the
- * pre-pass for its queries, recomputing S and dP), then dK/dV; a split call
- * adds one reduce of the partials.  Either way everything queued on `stream`
+ * pre-pass for its queries, recomputing S and dP), then dK/dV.  A split call
+ * adds one reduce of the partials.  Everything queued on `stream`
  * afterwards sees the results.  Replaces AttnBwd::bwd (lib.rs:216-263). */
 fa_status fa_attn_bwd(const fa_attn_bwd_args *args, void *stream);
 
@@ -214,7 +214,7 @@ fa_status fa_attn_bwd_phase(const fa_attn_bwd_args *args, int32_t phase, void *s
  * device code, one per GPU, held until the process ends, so calls with
  * B * heads * seq > FA_BWD_NOALLOC_MAX_ROWS fail with FA_ERR_INVALID_ARG.
  * The call never splits key or query ranges (the split partials would not
- * fit), runs every launch in order on `stream` (no side stream), and calls no
+ * fit), runs every launch in order on `stream`, and calls no
  * allocating routine.  For shapes fa_attn_bwd does not split the results are
  * bit-identical to fa_attn_bwd's; for shapes it splits they are the unsplit
  * kernels' results (deterministic, within the same tolerance of the exact
