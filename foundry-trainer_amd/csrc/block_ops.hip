@@ -45,6 +45,33 @@ __device__ __forceinline__ void store8(float *p, const float v[8]) {
     *reinterpret_cast<f32x4 *>(p + 4) = f32x4{v[4], v[5], v[6], v[7]};
 }
 
+// The same past the caches' allocation: for streams far larger than the L2s
+// that nothing reads again soon.
+__device__ __forceinline__ void load8nt(const bf16 *p, float v[8]) {
+    const bf16x8 a = as_bf16x8(__builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p)));
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = (float)a[j];
+}
+__device__ __forceinline__ void load8nt(const float *p, float v[8]) {
+    const f32x4 a = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(p));
+    const f32x4 b = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(p + 4));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        v[j] = a[j];
+        v[4 + j] = b[j];
+    }
+}
+__device__ __forceinline__ void store8nt(bf16 *p, const float v[8]) {
+    bf16x8 a;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) a[j] = f32_to_bf16(v[j]);
+    __builtin_nontemporal_store(as_u32x4(a), reinterpret_cast<u32x4 *>(p));
+}
+__device__ __forceinline__ void store8nt(float *p, const float v[8]) {
+    __builtin_nontemporal_store(f32x4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f32x4 *>(p));
+    __builtin_nontemporal_store(f32x4{v[4], v[5], v[6], v[7]}, reinterpret_cast<f32x4 *>(p + 4));
+}
+
 // x rounded to the storage type T, back in f32
 template <typename T>
 __device__ __forceinline__ float round_to(float x) {
@@ -224,7 +251,10 @@ __device__ __forceinline__ float gelu_sigmoid(float u) {
 }
 
 // Grid: x over 128-lane groups of a row's 8-element chunks, y over rows
-// (striding by gridDim.y), so no lane divides to find its row.
+// (striding by gridDim.y), so no lane divides to find its row.  Results, and
+// what the GELU gradient reads last, go past the caches: with GELU and its
+// gradient at 4096 x 9216 bf16 between the block's layer norms from cold HBM,
+// the four launches 114 -> 102 us.
 constexpr int kEltLanes = 128;
 template <typename T, int OP>
 __global__ __launch_bounds__(kEltLanes) void elementwise_kernel(EltParams p) {
@@ -233,7 +263,11 @@ __global__ __launch_bounds__(kEltLanes) void elementwise_kernel(EltParams p) {
     const T *g = static_cast<const T *>(p.g);
     for (int64_t row = blockIdx.y; row < p.N; row += gridDim.y) {
         float bv[8], o[8];
-        load8(static_cast<const T *>(p.b) + row * p.ldb + e, bv);
+        const T *b = static_cast<const T *>(p.b) + row * p.ldb + e;
+        if constexpr (OP == 2)
+            load8nt(b, bv);  // the pre-activation's last use
+        else
+            load8(b, bv);
         if constexpr (OP == 0) {
             float gv[8], xv[8];
             load8(g + e, gv);
@@ -250,7 +284,7 @@ __global__ __launch_bounds__(kEltLanes) void elementwise_kernel(EltParams p) {
             for (int j = 0; j < 8; ++j) o[j] = bv[j] * gelu_sigmoid(bv[j]);
         } else if constexpr (OP == 2) {
             float xv[8];
-            load8(static_cast<const T *>(p.x) + row * p.ldx + e, xv);
+            load8nt(static_cast<const T *>(p.x) + row * p.ldx + e, xv);
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const float u = bv[j];
@@ -262,7 +296,7 @@ __global__ __launch_bounds__(kEltLanes) void elementwise_kernel(EltParams p) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) o[j] = bv[j] / (1.f + exp2_fast(-kLog2e * bv[j]));
         }
-        store8(static_cast<T *>(p.y) + row * p.ldy + e, o);
+        store8nt(static_cast<T *>(p.y) + row * p.ldy + e, o);
     }
 }
 
@@ -270,22 +304,30 @@ __global__ __launch_bounds__(kEltLanes) void elementwise_kernel(EltParams p) {
 // * u).  Backward: du = T(dy * T(silu(g))), dg = T(T(dy * u) * silu'(g)) with
 // silu'(g) = s (1 + g (1 - s)), s = 1 / (1 + e^-g); T() = round to storage.
 // The grid is the elementwise kernel's (a form that strode over all elements
-// divided a 64-bit index by the row length on each): 4608 x 9216 bf16 from cold
-// HBM 54 -> 50 us forward, 81 -> 74 us backward (5.1, 5.7 TB/s).
+// divided a 64-bit index by the row length on each), and what the backward
+// reads last and both write goes past the caches: 4608 x 9216 bf16 from cold
+// HBM 54 -> 50 -> 44 us forward (5.8 TB/s), 81 -> 74 -> 63 us backward (6.7 TB/s),
+// and the layer-norm backward after it 27 -> 21.
 template <typename T, bool BWD>
 __global__ __launch_bounds__(kEltLanes) void swiglu_kernel(SwigluParams p) {
     const int e = (blockIdx.x * kEltLanes + threadIdx.x) * 8;
     if (e >= p.C) return;
     for (int64_t row = blockIdx.y; row < p.N; row += gridDim.y) {
         float gv[8], uv[8], o[8];
-        load8(static_cast<const T *>(p.gate) + row * p.ldg + e, gv);
-        load8(static_cast<const T *>(p.up) + row * p.ldu + e, uv);
+        const T *gate = static_cast<const T *>(p.gate) + row * p.ldg + e, *up = static_cast<const T *>(p.up) + row * p.ldu + e;
+        if constexpr (BWD) {
+            load8nt(gate, gv);
+            load8nt(up, uv);
+        } else {
+            load8(gate, gv);
+            load8(up, uv);
+        }
         if constexpr (!BWD) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) o[j] = round_to<T>(gv[j] / (1.f + exp2_fast(-kLog2e * gv[j]))) * uv[j];
         } else {
             float dv[8], du[8];
-            load8(static_cast<const T *>(p.dy) + row * p.lddy + e, dv);
+            load8nt(static_cast<const T *>(p.dy) + row * p.lddy + e, dv);
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const float g = gv[j];
@@ -294,9 +336,9 @@ __global__ __launch_bounds__(kEltLanes) void swiglu_kernel(SwigluParams p) {
                 du[j] = dv[j] * silu;
                 o[j] = round_to<T>(dv[j] * uv[j]) * (sg * (1.f + g * (1.f - sg)));
             }
-            store8(static_cast<T *>(p.dup) + row * p.lddup + e, du);
+            store8nt(static_cast<T *>(p.dup) + row * p.lddup + e, du);
         }
-        store8(static_cast<T *>(p.y) + row * p.ldy + e, o);
+        store8nt(static_cast<T *>(p.y) + row * p.ldy + e, o);
     }
 }
 
