@@ -7,7 +7,9 @@ the shared library is missing there is no fallback path.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
+import struct
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(os.path.dirname(_PKG_DIR), "libfoundry_attn.so")
@@ -279,6 +281,49 @@ def lib() -> ctypes.CDLL:
                                       ctypes.c_void_p, ctypes.c_void_p]
     _lib = L
     return L
+
+
+# ---------------------------------------------------------------------------
+# Calls by packed bytes.  Filling a ctypes structure field by field costs as
+# much host time as the shortest kernels run; packing the same layout with one
+# struct call and passing the bytes takes about a third of it.
+# ---------------------------------------------------------------------------
+_CODES = {ctypes.c_int32: "i", ctypes.c_int64: "q", ctypes.c_float: "f", ctypes.c_double: "d",
+          ctypes.c_void_p: "P", ctypes.c_size_t: "N"}
+
+
+def _codes(t) -> str:
+    if t in _CODES:
+        return _CODES[t]
+    if issubclass(t, ctypes.Array):
+        return _codes(t._type_) * t._length_
+    return "".join(_codes(f[1]) for f in t._fields_)
+
+
+def packer(cls):
+    """pack(values in field order, nested ones flattened, pointers as ints) ->
+    bytes laid out as the structure cls."""
+    st = struct.Struct("@" + _codes(cls) + "0q")
+    if st.size != ctypes.sizeof(cls):
+        raise AssertionError(f"{cls.__name__}: packed size {st.size}, structure {ctypes.sizeof(cls)}")
+    return st.pack
+
+
+@functools.lru_cache(maxsize=None)
+def entry(name: str, *argtypes, size: bool = False):
+    """Library function `name` taking packed arguments (bytes), then argtypes;
+    size: it returns a byte count, not a status."""
+    fn = lib()[name]  # a handle of its own: the attribute's keeps its structure types
+    fn.restype = ctypes.c_size_t if size else ctypes.c_int
+    fn.argtypes = [ctypes.c_char_p, *argtypes]
+    return fn
+
+
+def call(name: str, args: bytes, stream: int) -> None:
+    """fa_status name(args, stream), raising on an error status."""
+    status = entry(name, ctypes.c_void_p)(args, stream)
+    if status != FA_OK:
+        check(status)
 
 
 def check(status: int) -> None:

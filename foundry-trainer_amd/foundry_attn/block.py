@@ -45,7 +45,7 @@ import torch
 
 from . import _abi, gemm_tuning
 from ._abi import FoundryAttnError, check, lib
-from .ops import (_dtype_code, _ptr, _stream, attn_bwd, attn_bwd_workspace_bytes, attn_fwd, lora_bwd, lora_down,
+from .ops import (_dtype_code, _f32, _ptr, _stream, attn_bwd, attn_bwd_workspace_bytes, attn_fwd, lora_bwd, lora_down,
                   lora_fwd, lora_grad,
                   lora_grad_many,
                   lora_up, qk_prologue_bwd_multi, qk_prologue_multi, rope_tables)
@@ -54,6 +54,15 @@ from .ops import (_dtype_code, _ptr, _stream, attn_bwd, attn_bwd_workspace_bytes
 # ---------------------------------------------------------------------------
 # block ops (include/foundry_block.h)
 # ---------------------------------------------------------------------------
+_pack_ln = _abi.packer(_abi.LnModArgs)
+_pack_ln_bwd = _abi.packer(_abi.LnModBwdArgs)
+_pack_gated_ln = _abi.packer(_abi.GatedLnModArgs)
+_pack_ln_bwd_gate = _abi.packer(_abi.LnModBwdGateArgs)
+_pack_rows = _abi.packer(_abi.RowsArgs)
+_pack_swiglu = _abi.packer(_abi.SwigluArgs)
+_pack_swiglu_bwd = _abi.packer(_abi.SwigluBwdArgs)
+
+
 def _rows(t: torch.Tensor, name: str) -> torch.Tensor:
     if t.dim() != 2 or t.stride(1) != 1:
         raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG, f"{name} must be 2-D with contiguous rows")
@@ -86,11 +95,18 @@ def ln_mod_fwd(x, shift, scale, eps: float = 1e-6, out=None, stats: bool = False
     if stats:
         mean = torch.empty(N, dtype=torch.float32, device=x.device)
         rstd = torch.empty(N, dtype=torch.float32, device=x.device)
-    a = _abi.LnModArgs(dtype=_dtype_code(x), rows=N, cols=C, eps=float(eps), x=_ptr(x), ldx=x.stride(0),
-                       shift=_ptr(_vec(shift, C, x, "shift")), scale=_ptr(_vec(scale, C, x, "scale")),
-                       y=_ptr(y), ldy=y.stride(0), mean=_ptr(mean), rstd=_ptr(rstd))
-    check(lib().fa_ln_mod_fwd(ctypes.byref(a), _stream(x)))
+    a = _pack_ln(_dtype_code(x), N, C, _f32(eps), x.data_ptr(), x.stride(0), _vec(shift, C, x, "shift").data_ptr(),
+                 _vec(scale, C, x, "scale").data_ptr(), y.data_ptr(), y.stride(0), _ptr(mean),
+                 _ptr(rstd))
+    _abi.call("fa_ln_mod_fwd", a, _stream(x))
     return (y, mean, rstd) if stats else y
+
+
+def _ln_bwd_args(x, dy, scale, mean, rstd, eps, dres, dx) -> tuple:
+    """LnModBwdArgs' values in field order (the shift is not read)."""
+    sc = _vec(scale, x.shape[1], x, "scale").data_ptr()
+    return (_dtype_code(x), *x.shape, _f32(eps), x.data_ptr(), x.stride(0), sc, sc, 0, 0, _ptr(mean), _ptr(rstd),
+            dy.data_ptr(), dy.stride(0), _ptr(dres), 0 if dres is None else dres.stride(0), dx.data_ptr(), dx.stride(0))
 
 
 def ln_mod_bwd(x, dy, scale, mean, rstd, eps: float = 1e-6, dres=None, out=None):
@@ -100,12 +116,7 @@ def ln_mod_bwd(x, dy, scale, mean, rstd, eps: float = 1e-6, dres=None, out=None)
     dx = _like(out, x)
     if dres is not None:
         _rows(dres, "dres")
-    fwd = _abi.LnModArgs(dtype=_dtype_code(x), rows=N, cols=C, eps=float(eps), x=_ptr(x), ldx=x.stride(0),
-                         shift=_ptr(_vec(scale, C, x, "scale")), scale=_ptr(_vec(scale, C, x, "scale")),
-                         mean=_ptr(mean), rstd=_ptr(rstd))
-    a = _abi.LnModBwdArgs(fwd=fwd, dy=_ptr(dy), lddy=dy.stride(0), dres=_ptr(dres),
-                          ldres=0 if dres is None else dres.stride(0), dx=_ptr(dx), lddx=dx.stride(0))
-    check(lib().fa_ln_mod_bwd(ctypes.byref(a), _stream(x)))
+    _abi.call("fa_ln_mod_bwd", _pack_ln_bwd(*_ln_bwd_args(x, dy, scale, mean, rstd, eps, dres, dx)), _stream(x))
     return dx
 
 
@@ -123,13 +134,12 @@ def gated_ln_mod_fwd(x, g, b, shift, scale, eps: float = 1e-6, out=None, sum_out
         _like(sum_copy, x, "sum_copy")
     mean = torch.empty(N, dtype=torch.float32, device=x.device)
     rstd = torch.empty(N, dtype=torch.float32, device=x.device)
-    ln = _abi.LnModArgs(dtype=_dtype_code(x), rows=N, cols=C, eps=float(eps), x=_ptr(x), ldx=x.stride(0),
-                        shift=_ptr(_vec(shift, C, x, "shift")), scale=_ptr(_vec(scale, C, x, "scale")),
-                        y=_ptr(y), ldy=y.stride(0), mean=_ptr(mean), rstd=_ptr(rstd))
-    a = _abi.GatedLnModArgs(ln=ln, g=_ptr(_vec(g, C, x, "g")), b=_ptr(b), ldb=b.stride(0), sum=_ptr(s),
-                            ldsum=s.stride(0), sum2=_ptr(sum_copy),
-                            ldsum2=0 if sum_copy is None else sum_copy.stride(0))
-    check(lib().fa_gated_ln_mod_fwd(ctypes.byref(a), _stream(x)))
+    a = _pack_gated_ln(_dtype_code(x), N, C, _f32(eps), x.data_ptr(), x.stride(0),
+                       _vec(shift, C, x, "shift").data_ptr(), _vec(scale, C, x, "scale").data_ptr(), y.data_ptr(),
+                       y.stride(0), mean.data_ptr(), rstd.data_ptr(), _vec(g, C, x, "g").data_ptr(), b.data_ptr(),
+                       b.stride(0), s.data_ptr(), s.stride(0), _ptr(sum_copy),
+                       0 if sum_copy is None else sum_copy.stride(0))
+    _abi.call("fa_gated_ln_mod_fwd", a, _stream(x))
     return s, y, mean, rstd
 
 
@@ -142,13 +152,9 @@ def ln_mod_bwd_gate(x, dy, scale, mean, rstd, g, eps: float = 1e-6, dres=None, o
     gdx = _like(gated_out, x, "gated_out")
     if dres is not None:
         _rows(dres, "dres")
-    fwd = _abi.LnModArgs(dtype=_dtype_code(x), rows=N, cols=C, eps=float(eps), x=_ptr(x), ldx=x.stride(0),
-                         shift=_ptr(_vec(scale, C, x, "scale")), scale=_ptr(_vec(scale, C, x, "scale")),
-                         mean=_ptr(mean), rstd=_ptr(rstd))
-    bw = _abi.LnModBwdArgs(fwd=fwd, dy=_ptr(dy), lddy=dy.stride(0), dres=_ptr(dres),
-                           ldres=0 if dres is None else dres.stride(0), dx=_ptr(dx), lddx=dx.stride(0))
-    a = _abi.LnModBwdGateArgs(bwd=bw, g=_ptr(_vec(g, C, x, "g")), gdx=_ptr(gdx), ldgdx=gdx.stride(0))
-    check(lib().fa_ln_mod_bwd_gate(ctypes.byref(a), _stream(x)))
+    a = _pack_ln_bwd_gate(*_ln_bwd_args(x, dy, scale, mean, rstd, eps, dres, dx), _vec(g, C, x, "g").data_ptr(),
+                          gdx.data_ptr(), gdx.stride(0))
+    _abi.call("fa_ln_mod_bwd_gate", a, _stream(x))
     return dx, gdx
 
 
@@ -158,9 +164,9 @@ def _rows_op(fn, x, g, b, out):
     y = _like(out, b)
     if x is not None:
         _rows(x, "x")
-    a = _abi.RowsArgs(dtype=_dtype_code(b), rows=N, cols=C, x=_ptr(x), ldx=0 if x is None else x.stride(0),
-                      g=_ptr(g), b=_ptr(b), ldb=b.stride(0), y=_ptr(y), ldy=y.stride(0))
-    check(getattr(lib(), fn)(ctypes.byref(a), _stream(b)))
+    a = _pack_rows(_dtype_code(b), N, C, _ptr(x), 0 if x is None else x.stride(0), _ptr(g), b.data_ptr(), b.stride(0),
+                   y.data_ptr(), y.stride(0))
+    _abi.call(fn, a, _stream(b))
     return y
 
 
@@ -216,12 +222,11 @@ def _same_rows(t: torch.Tensor, ref: torch.Tensor, name: str) -> torch.Tensor:
     return t
 
 
-def _swiglu_args(gate, up):
+def _swiglu_args(gate, up) -> tuple:
+    """SwigluArgs' values in field order, up to y."""
     gate = _rows(gate, "gate")
     _same_rows(up, gate, "up")
-    N, C = gate.shape
-    return _abi.SwigluArgs(dtype=_dtype_code(gate), rows=N, cols=C, gate=_ptr(gate), ldgate=gate.stride(0),
-                           up=_ptr(up), ldup=up.stride(0))
+    return (_dtype_code(gate), *gate.shape, gate.data_ptr(), gate.stride(0), up.data_ptr(), up.stride(0))
 
 
 def swiglu(gate, up, out=None):
@@ -229,8 +234,7 @@ def swiglu(gate, up, out=None):
     may be column slices of one fused projection output."""
     a = _swiglu_args(gate, up)
     y = _like(out, gate)
-    a.y, a.ldy = _ptr(y), y.stride(0)
-    check(lib().fa_swiglu_fwd(ctypes.byref(a), _stream(gate)))
+    _abi.call("fa_swiglu_fwd", _pack_swiglu(*a, y.data_ptr(), y.stride(0)), _stream(gate))
     return y
 
 
@@ -239,9 +243,9 @@ def swiglu_bwd(dy, gate, up, dgate=None, dup=None):
     fwd = _swiglu_args(gate, up)
     _same_rows(dy, gate, "dy")
     dg, du = _like(dgate, gate, "dgate"), _like(dup, gate, "dup")
-    a = _abi.SwigluBwdArgs(fwd=fwd, dy=_ptr(dy), lddy=dy.stride(0), dgate=_ptr(dg), lddgate=dg.stride(0),
-                           dup=_ptr(du), lddup=du.stride(0))
-    check(lib().fa_swiglu_bwd(ctypes.byref(a), _stream(gate)))
+    a = _pack_swiglu_bwd(*fwd, 0, 0, dy.data_ptr(), dy.stride(0), dg.data_ptr(), dg.stride(0), du.data_ptr(),
+                         du.stride(0))
+    _abi.call("fa_swiglu_bwd", a, _stream(gate))
     return dg, du
 
 

@@ -40,10 +40,10 @@ def _dtype_code(t: torch.Tensor) -> int:
 
 
 def _as4(t: torch.Tensor, name: str) -> torch.Tensor:
-    if t.dim() == 3:
-        t = t.unsqueeze(0)
     if t.dim() != 4:
-        raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG, f"{name} must be (S,H,D) or (B,S,H,D)")
+        if t.dim() != 3:
+            raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG, f"{name} must be (S,H,D) or (B,S,H,D)")
+        t = t.unsqueeze(0)
     if not t.is_cuda:
         raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG, f"{name} must be a device tensor")
     if t.stride(3) != 1:
@@ -51,8 +51,9 @@ def _as4(t: torch.Tensor, name: str) -> torch.Tensor:
     return t
 
 
-def _strides(t: torch.Tensor) -> _abi.Strides:
-    return _abi.Strides(t.stride(0), t.stride(1), t.stride(2))
+def _strides(t: torch.Tensor) -> tuple:
+    """(batch, sequence, head) strides of a 4-D view."""
+    return t.stride()[:3]
 
 
 def _stream(t: torch.Tensor) -> int:
@@ -60,21 +61,40 @@ def _stream(t: torch.Tensor) -> int:
     device: the library launches on the current HIP device (and sizes split
     workspaces for it), so a tensor elsewhere is refused rather than read
     from the wrong GPU."""
-    cur = torch.cuda.current_device()
-    if t.device.index != cur:
+    dev, cur = t.get_device(), torch._C._cuda_getDevice()
+    if dev != cur:
         raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG,
                                f"{t.device} is not the current device cuda:{cur}; the library launches on the "
                                f"current device: call inside `with torch.cuda.device({t.device})`")
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(cur)
 
 
-def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
-    return None if t is None else t.data_ptr()
+def _ptr(t: Optional[torch.Tensor]) -> int:
+    return 0 if t is None else t.data_ptr()
+
+
+def _f32(x) -> float:
+    """x as the f32 field holds it (infinite past its range, for the library to refuse)."""
+    return ctypes.c_float(x).value
+
+
+_pack_fwd = _abi.packer(_abi.AttnFwdArgs)
+_pack_bwd = _abi.packer(_abi.AttnBwdArgs)
+_pack_prologue = _abi.packer(_abi.QkPrologueArgs)
+_pack_prologue_bwd = _abi.packer(_abi.QkPrologueBwdArgs)
+_pack_lora = _abi.packer(_abi.LoraArgs)
+_pack_lora_bwd = _abi.packer(_abi.LoraBwdArgs)
+_pack_lora_down = _abi.packer(_abi.LoraDownArgs)
+_pack_lora_up = _abi.packer(_abi.LoraUpArgs)
+_pack_lora_grad = _abi.packer(_abi.LoraGradArgs)
 
 
 def _keep(key_keep: Optional[torch.Tensor], B: int, S: int, dev) -> Optional[torch.Tensor]:
     if key_keep is None:
         return None
+    if key_keep.dtype == torch.uint8 and key_keep.shape == (B, S) and key_keep.device == dev \
+            and key_keep.is_contiguous():
+        return key_keep
     kk = key_keep.to(device=dev, dtype=torch.uint8).reshape(B, S).contiguous()
     return kk
 
@@ -108,17 +128,17 @@ def attn_fwd(q, k, v, scale: Optional[float] = None, key_keep=None, out=None, ls
             or lse_t.device != q4.device:
         raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG, "lse must be contiguous float32 (B,H,S)")
     kk = _keep(key_keep, B, S, q4.device)
-    a = _abi.AttnFwdArgs(dtype=_dtype_code(q4), batch=B, seq=S, heads=H, head_dim=D, scale=scale,
-                         q=_ptr(q4), k=_ptr(k4), v=_ptr(v4), o=_ptr(o4), lse=_ptr(lse_t),
-                         key_keep=_ptr(kk), q_stride=_strides(q4), k_stride=_strides(k4),
-                         v_stride=_strides(v4), o_stride=_strides(o4))
-    need = lib().fa_attn_fwd_workspace_size(ctypes.byref(a)) if split else 0
+    stream = _stream(q4)
+    head = (_dtype_code(q4), B, S, H, D, _f32(scale), q4.data_ptr(), k4.data_ptr(), v4.data_ptr(), o4.data_ptr(),
+            lse_t.data_ptr(), _ptr(kk), *_strides(q4), *_strides(k4), *_strides(v4),
+            *_strides(o4))
+    args = _pack_fwd(*head, 0, 0)
+    need = _abi.entry("fa_attn_fwd_workspace_size", size=True)(args) if split else 0
     if need:
         if workspace is None or workspace.numel() * workspace.element_size() < need:
             workspace = torch.empty(need, dtype=torch.uint8, device=q4.device)
-        a.workspace = workspace.data_ptr()
-        a.workspace_bytes = workspace.numel() * workspace.element_size()
-    check(lib().fa_attn_fwd(ctypes.byref(a), _stream(q4)))
+        args = _pack_fwd(*head, workspace.data_ptr(), workspace.numel() * workspace.element_size())
+    _abi.call("fa_attn_fwd", args, stream)
     return (o4[0] if squeeze else o4), lse_t
 
 
@@ -180,32 +200,34 @@ def attn_bwd(q, k, v, o, dout, lse, scale: Optional[float] = None, key_keep=None
     # (and out of the caching allocator) until it has been enqueued, or the
     # workspace allocated below could reuse its block
     lse_c = lse.contiguous()
-    a = _abi.AttnBwdArgs(dtype=_dtype_code(q4), batch=B, seq=S, heads=H, head_dim=D, scale=scale,
-                         q=_ptr(q4), k=_ptr(k4), v=_ptr(v4), o=_ptr(o4), dout=_ptr(do4),
-                         lse=_ptr(lse_c), key_keep=_ptr(kk), dq=_ptr(dq), dk=_ptr(dk),
-                         dv=_ptr(dv), q_stride=_strides(q4), k_stride=_strides(k4),
-                         v_stride=_strides(v4), o_stride=_strides(o4), do_stride=_strides(do4),
-                         dq_stride=_strides(dq), dk_stride=_strides(dk), dv_stride=_strides(dv))
+    stream = _stream(q4)
+    head = (_dtype_code(q4), B, S, H, D, _f32(scale), q4.data_ptr(), k4.data_ptr(), v4.data_ptr(), o4.data_ptr(),
+            do4.data_ptr(), lse_c.data_ptr(), _ptr(kk), dq.data_ptr(), dk.data_ptr(),
+            dv.data_ptr())
+    strides = (*_strides(q4), *_strides(k4), *_strides(v4), *_strides(o4), *_strides(do4), *_strides(dq),
+               *_strides(dk), *_strides(dv))
     # a given workspace of at least the minimum is used as it is (below the
     # full size: dQ recomputes S and dP); none gets the full size (dQ reads
     # the dK/dV kernel's stored dS)
-    need = lib().fa_attn_bwd_ds_workspace_size(ctypes.byref(a))
-    least = lib().fa_attn_bwd_min_workspace_size(ctypes.byref(a))
-    if workspace is None or workspace.numel() * workspace.element_size() < least:
+    given = 0 if workspace is None else workspace.numel() * workspace.element_size()
+    least = 0
+    if workspace is not None:
+        least = _abi.entry("fa_attn_bwd_min_workspace_size", size=True)(_pack_bwd(*head, 0, 0, *strides))
+    if workspace is None or given < least:
         if workspace is not None and phases is not None:
             # separate phase calls share the pre-pass rows through it
             raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG,
-                                   f"workspace of {workspace.numel() * workspace.element_size()} bytes is "
-                                   f"smaller than the {least} these shapes need")
-        workspace = torch.empty(max(need, 256), dtype=torch.uint8, device=q4.device)
-    a.workspace = workspace.data_ptr()
-    a.workspace_bytes = workspace.numel() * workspace.element_size()
+                                   f"workspace of {given} bytes is smaller than the {least} these shapes need")
+        need = _abi.entry("fa_attn_bwd_ds_workspace_size", size=True)(_pack_bwd(*head, 0, 0, *strides))
+        given = max(need, 256)
+        workspace = torch.empty(given, dtype=torch.uint8, device=q4.device)
+    args = _pack_bwd(*head, workspace.data_ptr(), given, *strides)
     if phases is None:
-        check(lib().fa_attn_bwd(ctypes.byref(a), _stream(q4)))
+        _abi.call("fa_attn_bwd", args, stream)
     else:
         for ph, st in phases:
-            sp = _stream(q4) if st is None else st.cuda_stream
-            check(lib().fa_attn_bwd_phase(ctypes.byref(a), int(ph), sp))
+            sp = stream if st is None else st.cuda_stream
+            check(_abi.entry("fa_attn_bwd_phase", ctypes.c_int32, ctypes.c_void_p)(args, int(ph), sp))
     del lse_c, kk  # enqueued: the stream orders any reuse of their blocks
     if squeeze:
         return dq[0], dk[0], dv[0]
@@ -331,23 +353,21 @@ def rope_tables(positions, axes: Sequence[int], theta: float, dtype=torch.bfloat
     return c.to(device), s.to(device)
 
 
-def _prologue_args(x4, weight, cos, sin, axes, eps, y4, seq_offset) -> _abi.QkPrologueArgs:
+def _prologue_args(x4, weight, cos, sin, axes, eps, y4, seq_offset) -> tuple:
+    """QkPrologueArgs' values in field order."""
     B, T, H, D = x4.shape
-    if len(axes) > _abi.FA_MAX_ROPE_AXES:
+    n = len(axes)
+    if n > _abi.FA_MAX_ROPE_AXES:
         raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG, "too many rope axes")
-    ax = (ctypes.c_int32 * _abi.FA_MAX_ROPE_AXES)(*([int(a) for a in axes] +
-                                                    [0] * (_abi.FA_MAX_ROPE_AXES - len(axes))))
+    dt, dev = x4.dtype, x4.device
     for name, t in (("weight", weight), ("cos", cos), ("sin", sin)):
-        if t.dtype != x4.dtype or not t.is_contiguous() or t.device != x4.device:
-            raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG,
-                                   f"{name} must be a contiguous {x4.dtype} tensor on {x4.device}")
+        if t.dtype != dt or not t.is_contiguous() or t.device != dev:
+            raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG, f"{name} must be a contiguous {dt} tensor on {dev}")
     if cos.shape != (T, D) or sin.shape != (T, D) or weight.shape != (D,):
         raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG, "weight/cos/sin shapes do not match x")
-    return _abi.QkPrologueArgs(dtype=_dtype_code(x4), batch=B, tokens=T, heads=H, head_dim=D,
-                               eps=float(eps), x=_ptr(x4), x_stride=_strides(x4),
-                               weight=_ptr(weight), cos=_ptr(cos), sin=_ptr(sin),
-                               n_axes=len(axes), axes=ax, y=_ptr(y4), y_stride=_strides(y4),
-                               y_seq_offset=int(seq_offset))
+    return (_dtype_code(x4), B, T, H, D, _f32(eps), x4.data_ptr(), *_strides(x4), weight.data_ptr(), cos.data_ptr(),
+            sin.data_ptr(), n, *map(int, axes), *(0,) * (_abi.FA_MAX_ROPE_AXES - n), y4.data_ptr(), *_strides(y4),
+            int(seq_offset))
 
 
 def _prologue_fwd_args(x, weight, cos, sin, axes, eps, out, seq_offset):
@@ -368,7 +388,7 @@ def qk_prologue(x, weight, cos, sin, axes: Sequence[int], eps: float = 1e-6,
     (B,S,H,D) buffer (allocated as (B,T,H,D) if None).  Returns out.
     """
     a, x4, y4 = _prologue_fwd_args(x, weight, cos, sin, axes, eps, out, seq_offset)
-    check(lib().fa_qk_prologue_fwd(ctypes.byref(a), _stream(x4)))
+    _abi.call("fa_qk_prologue_fwd", _pack_prologue(*a), _stream(x4))
     if out is None and x.dim() == 3:
         return y4[0]
     return out if out is not None else y4
@@ -383,8 +403,8 @@ def qk_prologue_multi(segments, eps: float = 1e-6):
     segs = [_prologue_fwd_args(x, w, c, s_, ax, eps, out, off) for (x, w, c, s_, ax, out, off) in segments]
     if not 1 <= len(segs) <= 4:
         raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG, "1..4 segments")
-    arr = (_abi.QkPrologueArgs * len(segs))(*[a for a, _, _ in segs])
-    check(lib().fa_qk_prologue_fwd_multi(arr, len(segs), _stream(segs[0][1])))
+    arr = b"".join([_pack_prologue(*a) for a, _, _ in segs])
+    check(_abi.entry("fa_qk_prologue_fwd_multi", ctypes.c_int32, ctypes.c_void_p)(arr, len(segs), _stream(segs[0][1])))
 
 
 def _prologue_bwd_args(x, weight, cos, sin, axes, dy, seq_offset, eps, dx):
@@ -399,8 +419,8 @@ def _prologue_bwd_args(x, weight, cos, sin, axes, dy, seq_offset, eps, dx):
         dx = _as4(dx, "dx")
         if dx.shape != x4.shape or dx.dtype != x4.dtype or dx.device != x4.device:
             raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG, "dx must match x")
-    a = _abi.QkPrologueBwdArgs(fwd=_prologue_args(x4, weight, cos, sin, axes, eps, dy4, seq_offset),
-                               dy=_ptr(dy4), dx=_ptr(dx), dx_stride=_strides(dx))
+    a = (*_prologue_args(x4, weight, cos, sin, axes, eps, dy4, seq_offset), dy4.data_ptr(), dx.data_ptr(),
+         *_strides(dx))
     return a, x4, dx
 
 
@@ -409,7 +429,7 @@ def qk_prologue_bwd(x, weight, cos, sin, axes: Sequence[int], dy, seq_offset: in
     """Gradient wrt x of qk_prologue, given dy wrt the joint buffer; written to
     `dx` (a view shaped like x, any row strides) when given."""
     a, x4, dx = _prologue_bwd_args(x, weight, cos, sin, axes, dy, seq_offset, eps, dx)
-    check(lib().fa_qk_prologue_bwd(ctypes.byref(a), _stream(x4)))
+    _abi.call("fa_qk_prologue_bwd", _pack_prologue_bwd(*a), _stream(x4))
     return dx[0] if x.dim() == 3 else dx
 
 
@@ -422,14 +442,15 @@ def qk_prologue_bwd_multi(segments, eps: float = 1e-6):
     segs = [_prologue_bwd_args(x, w, c, s_, ax, dy, off, eps, dx) for (x, w, c, s_, ax, dy, off, dx) in segments]
     if not 1 <= len(segs) <= 4:
         raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG, "1..4 segments")
-    arr = (_abi.QkPrologueBwdArgs * len(segs))(*[a for a, _, _ in segs])
-    check(lib().fa_qk_prologue_bwd_multi(arr, len(segs), _stream(segs[0][1])))
+    arr = b"".join([_pack_prologue_bwd(*a) for a, _, _ in segs])
+    check(_abi.entry("fa_qk_prologue_bwd_multi", ctypes.c_int32, ctypes.c_void_p)(arr, len(segs), _stream(segs[0][1])))
 
 
 # ---------------------------------------------------------------------------
 # LoRA
 # ---------------------------------------------------------------------------
-def _lora_args(x, a, b, y, scale, u) -> _abi.LoraArgs:
+def _lora_args(x, a, b, y, scale, u) -> tuple:
+    """LoraArgs' values in field order."""
     if x.dim() != 2 or a.dim() != 2 or b.dim() != 2:
         raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG, "x, lora_a, lora_b must be 2-D")
     N, K = x.shape
@@ -446,16 +467,14 @@ def _lora_args(x, a, b, y, scale, u) -> _abi.LoraArgs:
     if y is not None and (y.shape != (N, M) or y.stride(1) != 1 or y.dtype != x.dtype
                           or y.device != x.device):
         raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG, "y must be [N, M] with contiguous rows")
-    return _abi.LoraArgs(dtype=_dtype_code(x), tokens=N, in_features=K, out_features=M, rank=r,
-                         scale=float(scale), x=_ptr(x), ldx=x.stride(0), a=_ptr(a), b=_ptr(b),
-                         u=_ptr(u), y=_ptr(y), ldy=0 if y is None else y.stride(0))
+    return (_dtype_code(x), N, K, M, r, _f32(scale), x.data_ptr(), x.stride(0), a.data_ptr(), b.data_ptr(),
+            u.data_ptr(), _ptr(y), 0 if y is None else y.stride(0))
 
 
 def lora_fwd(x, a, b, y, scale: float):
     """y += scale * (x a^T) b^T in place; returns u = x a^T (f32) for the backward."""
     u = torch.empty((x.shape[0], a.shape[0]), dtype=torch.float32, device=x.device)
-    args = _lora_args(x, a, b, y, scale, u)
-    check(lib().fa_lora_fwd(ctypes.byref(args), _stream(x)))
+    _abi.call("fa_lora_fwd", _pack_lora(*_lora_args(x, a, b, y, scale, u)), _stream(x))
     return u
 
 
@@ -471,13 +490,11 @@ def lora_bwd(x, a, b, u, dy, scale: float, dx: Optional[torch.Tensor] = None):
         raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG, "dx must be [N, K] with contiguous rows")
     da = torch.empty((r, K), dtype=torch.float32, device=x.device)
     db = torch.empty((M, r), dtype=torch.float32, device=x.device)
-    args = _abi.LoraBwdArgs(fwd=_lora_args(x, a, b, None, scale, u), dy=_ptr(dy), ldy=dy.stride(0),
-                            da=_ptr(da), db=_ptr(db), dx=_ptr(dx),
-                            ldx=0 if dx is None else dx.stride(0))
-    need = lib().fa_lora_bwd_workspace_size(ctypes.byref(args))
+    head = (*_lora_args(x, a, b, None, scale, u), dy.data_ptr(), dy.stride(0), da.data_ptr(), db.data_ptr(),
+            _ptr(dx), 0 if dx is None else dx.stride(0))
+    need = _abi.entry("fa_lora_bwd_workspace_size", size=True)(_pack_lora_bwd(*head, 0, 0))
     ws = torch.empty(max(need, 256), dtype=torch.uint8, device=x.device)
-    args.workspace, args.workspace_bytes = ws.data_ptr(), ws.numel()
-    check(lib().fa_lora_bwd(ctypes.byref(args), _stream(x)))
+    _abi.call("fa_lora_bwd", _pack_lora_bwd(*head, ws.data_ptr(), ws.numel()), _stream(x))
     return da, db
 
 
@@ -518,9 +535,8 @@ def lora_down(x, a, scale: float, out: torch.Tensor):
     r = a.shape[0]
     a_c = _factor(a, (r, K), "lora_a", x)
     _rank_view(out, N, r, "out", x.device)
-    args = _abi.LoraDownArgs(dtype=_dtype_code(x), tokens=N, in_features=K, rank=r, scale=float(scale),
-                             x=_ptr(x), ldx=x.stride(0), a=_ptr(a_c), u=_ptr(out), ldu=out.stride(0))
-    check(lib().fa_lora_down(ctypes.byref(args), _stream(x)))
+    _abi.call("fa_lora_down", _pack_lora_down(_dtype_code(x), N, K, r, _f32(scale), x.data_ptr(), x.stride(0),
+                                              a_c.data_ptr(), out.data_ptr(), out.stride(0)), _stream(x))
     return out
 
 
@@ -534,14 +550,14 @@ def lora_up(u, b, y, scale: float):
     r = b.shape[1]
     b_c = _factor(b, (M, r), "lora_b", y)
     _rank_view(u, N, r, "u", y.device)
-    args = _abi.LoraUpArgs(dtype=_dtype_code(y), tokens=N, out_features=M, rank=r, scale=float(scale),
-                           u=_ptr(u), ldu=u.stride(0), b=_ptr(b_c), y=_ptr(y), ldy=y.stride(0))
-    check(lib().fa_lora_up(ctypes.byref(args), _stream(y)))
+    _abi.call("fa_lora_up", _pack_lora_up(_dtype_code(y), N, M, r, _f32(scale), u.data_ptr(), u.stride(0),
+                                          b_c.data_ptr(), y.data_ptr(), y.stride(0)), _stream(y))
     return y
 
 
 def _lora_grad_args(u, x, scale: float, transpose: bool, out: Optional[torch.Tensor]):
-    """Validated LoraGradArgs (no workspace yet) and the f32 output tensor."""
+    """Validated LoraGradArgs' values in field order, up to the workspace, and
+    the f32 output tensor."""
     x = _rows(x, "x", torch.bfloat16)
     N, C = x.shape
     if u.dim() != 2:
@@ -557,8 +573,8 @@ def _lora_grad_args(u, x, scale: float, transpose: bool, out: Optional[torch.Ten
             raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG,
                                    f"out must be a contiguous float32 {list(shape)} tensor on {x.device}")
         g = out
-    args = _abi.LoraGradArgs(dtype=_dtype_code(x), tokens=N, features=C, rank=r, scale=float(scale), u=_ptr(u),
-                             ldu=u.stride(0), x=_ptr(x), ldx=x.stride(0), grad=_ptr(g), transpose=int(transpose))
+    args = (_dtype_code(x), N, C, r, _f32(scale), u.data_ptr(), u.stride(0), x.data_ptr(), x.stride(0), g.data_ptr(),
+            int(transpose))
     return args, g
 
 
@@ -567,10 +583,9 @@ def lora_grad(u, x, scale: float, transpose: bool, out: Optional[torch.Tensor] =
     (lora_b layout).  u a bf16 [N, r] view, x [N, C] bf16 rows; `out`, when
     given, a contiguous f32 tensor of that shape on x's device."""
     args, g = _lora_grad_args(u, x, scale, transpose, out)
-    need = lib().fa_lora_grad_workspace_size(ctypes.byref(args))
+    need = _abi.entry("fa_lora_grad_workspace_size", size=True)(_pack_lora_grad(*args, 0, 0))
     ws = torch.empty(max(need, 256), dtype=torch.uint8, device=g.device)
-    args.workspace, args.workspace_bytes = ws.data_ptr(), ws.numel()
-    check(lib().fa_lora_grad(ctypes.byref(args), _stream(g)))
+    _abi.call("fa_lora_grad", _pack_lora_grad(*args, ws.data_ptr(), ws.numel()), _stream(g))
     return g
 
 
@@ -585,8 +600,9 @@ def lora_grad_many(items):
     dev = built[0][1].device
     if any(g.device != dev for _, g in built):
         raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG, "all products must be on one device")
-    arr = (_abi.LoraGradArgs * len(built))(*[a for a, _ in built])
-    need = lib().fa_lora_grad_many_workspace_size(arr, len(built))
+    arr = b"".join([_pack_lora_grad(*a, 0, 0) for a, _ in built])
+    need = _abi.entry("fa_lora_grad_many_workspace_size", ctypes.c_int32, size=True)(arr, len(built))
     ws = torch.empty(max(need, 256), dtype=torch.uint8, device=dev)
-    check(lib().fa_lora_grad_many(arr, len(built), ws.data_ptr(), ws.numel(), _stream(built[0][1])))
+    check(_abi.entry("fa_lora_grad_many", ctypes.c_int32, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p)(
+        arr, len(built), ws.data_ptr(), ws.numel(), _stream(built[0][1])))
     return [g for _, g in built]
