@@ -835,15 +835,32 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_bwd_dq_bf16_kernel(AttnBwdPar
 }
 
 // dK/dV and dQ of 4-wave shapes in one grid, after the pre-pass: the longer
-// dK/dV workgroups first, dQ's fill the CUs they leave.  (They are independent
-// after the pre-pass; 8-wave workgroups each fill a CU and stay separate.)
+// dK/dV workgroups first, dQ's fill the CUs they leave, but for q1 of them
+// brought forward to after the first d1 of dK/dV (pair_order).  (They are
+// independent after the pre-pass; 8-wave workgroups each fill a CU and stay
+// separate.)
 template <int D, bool KEEP>
-__global__ __launch_bounds__(256, 2) void attn_bwd_pair_bf16_kernel(AttnBwdParams p, int n_dkdv) {
+__global__ __launch_bounds__(256, 2) void attn_bwd_pair_bf16_kernel(AttnBwdParams p, int n, int d1, int q1) {
     const int b = blockIdx.x;
-    if (b < n_dkdv)
-        dkdv_block<D, 4, false, false, true>(p, xcd_remap(b, n_dkdv));
+    if (b < d1 || (b >= d1 + q1 && b < n + q1))
+        dkdv_block<D, 4, false, false, true>(p, xcd_remap(b < d1 ? b : b - q1, n));
     else
-        dq_block<D, KEEP, 4, false, false>(p, xcd_remap(b - n_dkdv, (int)gridDim.x - n_dkdv));
+        dq_block<D, KEEP, 4, false, false>(p, xcd_remap(b < d1 + q1 ? b - d1 : b - n, n));
+}
+
+// Order of the pair grid's 2n workgroups.  At D = 128 the chip holds w = 2 per
+// CU, and a dK/dV workgroup takes about 1.4 times as long as one of dQ.  With
+// n a little over w, dK/dV first leaves a second round of few dK/dV workgroups
+// and after it a third of few dQ.  Instead 5/8 of the places run two rounds of
+// dK/dV while 3/8 run three of dQ: what is left, n - 6w/8, fits those 3/8 and
+// the dK/dV places free after one round up to n = 19w/16 (608).  B2 H24 S1536
+// (n = 576) 222 -> 210 us, B4 S700 124 -> 117, B2 S1400 (528) 204 -> 190, B1
+// H25 S3072 (600) 434 -> 398; past the line H26 S3072 (624) 438 -> 466.  At D = 64
+// (3 per CU) no order gained more than 2%.
+void pair_order(int D, int n, int &d1, int &q1) {
+    const int w = 2 * device_cu_count();
+    d1 = n, q1 = 0;
+    if (D == 128 && n > w && 16 * n <= 19 * w) d1 = 5 * w / 8 & ~7, q1 = 6 * w / 8 & ~7;  // whole rounds of XCDs
 }
 
 template <int D, int NW, bool DELTA, bool SPLIT>
@@ -988,14 +1005,16 @@ hipError_t launch_attn_bwd_bf16(const AttnBwdParams &p, int D, int phase, hipStr
     }
     if (pair) {
         const dim3 pgrid(2 * n);
+        int d1, q1;
+        pair_order(D, n, d1, q1);
         if (D == 128 && p.keep)
-            hipLaunchKernelGGL((attn_bwd_pair_bf16_kernel<128, true>), pgrid, block, 0, s, p, n);
+            hipLaunchKernelGGL((attn_bwd_pair_bf16_kernel<128, true>), pgrid, block, 0, s, p, n, d1, q1);
         else if (D == 128)
-            hipLaunchKernelGGL((attn_bwd_pair_bf16_kernel<128, false>), pgrid, block, 0, s, p, n);
+            hipLaunchKernelGGL((attn_bwd_pair_bf16_kernel<128, false>), pgrid, block, 0, s, p, n, d1, q1);
         else if (p.keep)
-            hipLaunchKernelGGL((attn_bwd_pair_bf16_kernel<64, true>), pgrid, block, 0, s, p, n);
+            hipLaunchKernelGGL((attn_bwd_pair_bf16_kernel<64, true>), pgrid, block, 0, s, p, n, d1, q1);
         else
-            hipLaunchKernelGGL((attn_bwd_pair_bf16_kernel<64, false>), pgrid, block, 0, s, p, n);
+            hipLaunchKernelGGL((attn_bwd_pair_bf16_kernel<64, false>), pgrid, block, 0, s, p, n, d1, q1);
         return hipGetLastError();
     }
     if (fused || phase == 3) {

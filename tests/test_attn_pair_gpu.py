@@ -1,6 +1,7 @@
 """The one-grid dK/dV + dQ of the 4-wave bf16 backward: the bits of the two
 kernels issued as separate phases, over tile remainders, masks, D = 64 on
-grids where D = 128 takes 8 waves, and grids the range split leaves alone."""
+grids where D = 128 takes 8 waves, grids the range split leaves alone, and
+both ends of the sizes whose workgroups are reordered."""
 import pytest
 import torch
 
@@ -12,7 +13,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("masked", [False, True])
 @pytest.mark.parametrize("B,S,H,D", [(1, 1, 1, 128), (2, 129, 3, 128), (1, 511, 5, 64), (1, 700, 24, 128),
-                                     (1, 1100, 44, 64), (1, 1100, 4, 128), (1, 1024, 24, 64)])
+                                     (1, 1100, 44, 64), (1, 1100, 4, 128), (1, 1024, 24, 64),
+                                     (1, 128, 512, 128), (1, 100, 513, 128), (1, 128, 608, 128),
+                                     (1, 70, 609, 128), (2, 1400, 24, 128), (1, 100, 520, 64)])
 def test_pair_matches_phases(B, S, H, D, masked):
     torch.manual_seed(S + H)
     q, k, v, do = (torch.randn(B, S, H, D, device="cuda").to(torch.bfloat16) for _ in range(4))
