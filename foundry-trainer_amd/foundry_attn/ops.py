@@ -208,7 +208,8 @@ def attn_bwd(q, k, v, o, dout, lse, scale: Optional[float] = None, key_keep=None
                *_strides(dk), *_strides(dv))
     # a given workspace of at least the minimum is used as it is (below the
     # full size: dQ recomputes S and dP); none gets the full size (dQ reads
-    # the dK/dV kernel's stored dS)
+    # the dK/dV kernel's stored dS), or the minimum where memory has no room
+    # for the dS (up to FA_BWD_DS_MAX_BYTES): the same bits
     given = 0 if workspace is None else workspace.numel() * workspace.element_size()
     least = 0
     if workspace is not None:
@@ -220,7 +221,12 @@ def attn_bwd(q, k, v, o, dout, lse, scale: Optional[float] = None, key_keep=None
                                    f"workspace of {given} bytes is smaller than the {least} these shapes need")
         need = _abi.entry("fa_attn_bwd_ds_workspace_size", size=True)(_pack_bwd(*head, 0, 0, *strides))
         given = max(need, 256)
-        workspace = torch.empty(given, dtype=torch.uint8, device=q4.device)
+        try:
+            workspace = torch.empty(given, dtype=torch.uint8, device=q4.device)
+        except torch.cuda.OutOfMemoryError:
+            least = least or _abi.entry("fa_attn_bwd_min_workspace_size", size=True)(_pack_bwd(*head, 0, 0, *strides))
+            given = max(least, 256)
+            workspace = torch.empty(given, dtype=torch.uint8, device=q4.device)
     args = _pack_bwd(*head, workspace.data_ptr(), given, *strides)
     if phases is None:
         _abi.call("fa_attn_bwd", args, stream)

@@ -50,6 +50,30 @@ def test_groups_and_remainders(B, S, H, D):
             assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("dtype,S,H", [(torch.float32, 300, 4), (torch.bfloat16, 4608, 24)])
+def test_backward_without_room_for_ds(monkeypatch, dtype, S, H):
+    """Where memory has no room for the stored dS, the recomputing dQ runs: the same bits."""
+    gen = torch.Generator(device="cuda").manual_seed(S)
+    q, k, v, do = (torch.randn(1, S, H, 128, device="cuda", generator=gen).to(dtype) for _ in range(4))
+    o, lse = attn_fwd(q, k, v)
+    want = attn_bwd(q, k, v, o, do, lse)
+    least = attn_bwd_workspace_bytes(1, S, H, 128, dtype, minimum=True)
+    assert attn_bwd_workspace_bytes(1, S, H, 128, dtype) > least
+    empty, refused = torch.empty, []
+
+    def limited(*shape, **kw):
+        if kw.get("dtype") == torch.uint8 and shape[0] > least:
+            refused.append(shape[0])
+            raise torch.cuda.OutOfMemoryError("no room")
+        return empty(*shape, **kw)
+
+    monkeypatch.setattr(torch, "empty", limited)
+    got = attn_bwd(q, k, v, o, do, lse)
+    assert refused
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("D", [64, 128])
 def test_row_stride_past_32_bit_offsets(D):
     """Rows 2^25 elements apart: a 32-row tile spans 4 GiB and more."""
