@@ -138,6 +138,7 @@ struct LoraGradItem {
     float scale;
     float *grad;
     bool transpose;
+    int splits = 0;  // of the tokens; 0: by the product's own size
 };
 size_t lora_grad_many_workspace_bytes(const LoraGradItem *items, int count);
 hipError_t launch_lora_grad_many_bf16(const LoraGradItem *items, int count, void *work, hipStream_t st);

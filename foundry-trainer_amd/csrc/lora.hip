@@ -1047,6 +1047,22 @@ inline int colsum_splits(int N, int C) {
     if (sp > stages / (1024 / kCsRows)) sp = stages / (1024 / kCsRows);  // splits of >= 1024 tokens
     return sp < 1 ? 1 : sp;
 }
+// One adapter's two gradients alone in their launches (lora_bwd), `tiles`
+// column tiles in all.  Nothing else fills the chip here, so workgroups in
+// flight matter more than long splits: about 768 (three per CU), a split at
+// least 128 tokens (4 stages) long.  lora_bwd with dx, r 16, graph-replayed, us
+// for the splits above / 384 wgs of >= 512 tokens / 768 of >= 128 / 1536 of
+// >= 128: 4096 x 3072 x 3072 52.4 / 43.5 / 41.6 / 48.4, 4608 x 768 x 3072 48.2 /
+// 37.0 / 34.0 / 36.8, 1536 x 3072 x 3072 38.0 / 26.7 / 25.4 / 25.5, 600 x 3072 x
+// 768 22.7 / 22.8 / 19.1 / 19.1.
+constexpr int kBwdWgs = 768, kBwdTokens = 128;
+inline int colsum_bwd_splits(int N, int tiles) {
+    int sp = (kBwdWgs + tiles - 1) / tiles;
+    const int most = N / kBwdTokens;
+    sp = sp < most ? sp : most;
+    return sp < 1 ? 1 : sp;
+}
+inline int colsum_tiles(int K, int M) { return (K + kCsCols - 1) / kCsCols + (M + kCsCols - 1) / kCsCols; }
 inline int colsum_npad(int N) { return (N + kCsRows - 1) / kCsRows * kCsRows; }
 
 // Token splits of the f32 colsum: about 512 workgroups over both products
@@ -1062,9 +1078,8 @@ inline int colsum_f32_tiles(int K, int M) { return (K + 127) / 128 + (M + 127) /
 
 inline size_t al256(size_t x) { return (x + 255) & ~size_t(255); }
 inline int grad_rows(int R) { return R > 32 ? 64 : 32; }
-inline size_t grad_item_bytes(int N, int C, int R) {
-    return al256((size_t)grad_rows(R) * colsum_npad(N) * 2) +
-           al256((size_t)colsum_splits(N, C) * C * grad_rows(R) * 4);
+inline size_t grad_item_bytes(int N, int C, int R, int splits) {
+    return al256((size_t)grad_rows(R) * colsum_npad(N) * 2) + al256((size_t)splits * C * grad_rows(R) * 4);
 }
 
 hipError_t lora_fwd_bf16(const LoraParams &p, hipStream_t st) {
@@ -1157,8 +1172,9 @@ hipError_t lora_bwd_f32(const LoraParams &p, hipStream_t st) {
 // where it is formed: every product it enters rounds it to bf16.
 inline int bwd_ldub(int r) { return (r + 7) & ~7; }
 inline size_t lora_bwd_bf16_bytes(int N, int K, int M, int r) {
+    const int sp = colsum_bwd_splits(N, colsum_tiles(K, M));
     return 2 * al256((size_t)N * bwd_ldub(r) * 2) + al256((size_t)r * M * 2) + al256((size_t)K * r * 2) +
-           grad_item_bytes(N, M, r) + grad_item_bytes(N, K, r);
+           grad_item_bytes(N, M, r, sp) + grad_item_bytes(N, K, r, sp);
 }
 }  // namespace
 
@@ -1181,8 +1197,9 @@ static hipError_t lora_bwd_bf16(const LoraParams &p, hipStream_t st) {
     const bf16 *dy = static_cast<const bf16 *>(p.dy);
     if ((e = rowdot16<bf16, bf16>(dy, p.lddy, bt, du, ld, p.N, p.M, p.r, p.scale, st)) != hipSuccess) return e;
     // dB[o][j] = s * sum_n dy[n][o] u[n][j], dA[j][k] = sum_n du[n][j] x[n][k]
-    const LoraGradItem items[2] = {{ub, ld, p.dy, p.lddy, p.N, p.M, p.r, p.scale, p.db, true},
-                                   {du, ld, p.x, p.ldx, p.N, p.K, p.r, 1.f, p.da, false}};
+    const int sp = colsum_bwd_splits(p.N, colsum_tiles(p.K, p.M));
+    const LoraGradItem items[2] = {{ub, ld, p.dy, p.lddy, p.N, p.M, p.r, p.scale, p.db, true, sp},
+                                   {du, ld, p.x, p.ldx, p.N, p.K, p.r, 1.f, p.da, false, sp}};
     if ((e = launch_lora_grad_many_bf16(items, 2, ws, st)) != hipSuccess || !p.dx) return e;
     // dx += du A  (A^T [K, r] as Wt)
     return expand_mfma<bf16>(du, ld, at, static_cast<bf16 *>(p.dx), p.lddx, p.N, p.K, p.r, 1.f, st);
@@ -1219,7 +1236,7 @@ size_t lora_grad_many_workspace_bytes(const LoraGradItem *items, int count) {
     for (int k0 = 0; k0 < count; k0 += kGradMany) {
         size_t b = 0;
         for (int k = k0; k < count && k < k0 + kGradMany; ++k)
-            b += grad_item_bytes(items[k].N, items[k].C, items[k].R);
+            b += grad_item_bytes(items[k].N, items[k].C, items[k].R, colsum_splits(items[k].N, items[k].C));
         most = b > most ? b : most;
     }
     return most;
@@ -1250,8 +1267,9 @@ hipError_t launch_lora_grad_many_bf16(const LoraGradItem *items, int count, void
             q.rw = grad_rows(it.R);
             q.N = it.N;
             q.npad = colsum_npad(it.N);
-            q.splits = colsum_splits(it.N, it.C);
+            q.splits = it.splits ? it.splits : colsum_splits(it.N, it.C);
             q.chunk = (q.npad / kCsRows + q.splits - 1) / q.splits * kCsRows;
+            q.splits = (q.npad + q.chunk - 1) / q.chunk;  // none empty
             q.wg0 = wgs;
             q.ut = reinterpret_cast<bf16 *>(ws);
             ws += al256((size_t)q.rw * q.npad * 2);

@@ -222,6 +222,26 @@ def test_lora_bf16_ranks_ragged(r):
     assert rel_l2(host(dx), want_dx) <= 1e-2
 
 
+@pytest.mark.parametrize("N,K,M", [(31, 256, 256), (255, 256, 768), (256, 256, 256), (1000, 768, 256), (4607, 256, 256),
+                                   (1023, 3072, 3072)])
+@pytest.mark.parametrize("r", [4, 16])
+def test_lora_bwd_token_splits(N, K, M, r):
+    """Both gradients at one token split, at several, and with a short last
+    one.  The products' operands are bf16 (u and du rounded where they enter),
+    the sums f32: dB is off by f32 rounding only (N 2^-24 at most), dA by du's
+    rounding to bf16, 2^-9 at most."""
+    g = torch.Generator(device="cuda").manual_seed(N + r)
+    x, dy, a, b = (torch.randn(*sh, device="cuda", generator=g).to(torch.bfloat16)
+                   for sh in ((N, K), (N, M), (r, K), (M, r)))
+    u = torch.randn(N, r, device="cuda", generator=g)
+    da, db = lora_bwd(x, a, b, u, dy, 0.5)
+    x, dy, b = x.double(), dy.double(), b.double()
+    want_b = 0.5 * dy.t() @ u.to(torch.bfloat16).double()
+    want_a = (0.5 * dy @ b).t() @ x
+    assert rel_l2(host(db), host(want_b)) <= max(N, 16) * 2.0 ** -24
+    assert rel_l2(host(da), host(want_a)) <= 2.0 ** -9
+
+
 @pytest.mark.parametrize("K", [16, 208, 3088])
 @pytest.mark.parametrize("r", [16, 33, 48, 64])
 def test_lora_down_k_tails(K, r):
