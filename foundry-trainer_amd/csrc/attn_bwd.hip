@@ -982,7 +982,7 @@ hipError_t launch_attn_bwd_ds(const AttnBwdParams &p, int phase, hipStream_t s) 
     return e;
 }
 
-// Workgroup shape as for the forward (attn_waves) at D = 128.  At D = 64 4
+// Workgroup shape by attn_waves at D = 128.  At D = 64 4
 // waves throughout: the kernels' registers let three waves share a SIMD, and
 // dK/dV and dQ run in one grid (B1 H24 S4608 D64 562 -> 471 us, B4 S1536 281
 // -> 213, B1 S1536 88 -> 70).

@@ -502,8 +502,9 @@ int device_cu_count() {
     return n;
 }
 
-// Workgroup shape of the unsplit bf16 kernels (the backward's at D = 128; at D
-// = 64 it takes 4 waves throughout, see launch_attn_bwd_bf16).  An
+// Workgroup shape of the unsplit bf16 kernels (the forward's but for fwd_waves
+// below; the backward's at D = 128, which at D = 64 takes 4 waves throughout,
+// see launch_attn_bwd_bf16).  An
 // 8-wave workgroup fills a CU's registers alone (2 waves per SIMD), so its
 // grid runs in whole-CU rounds; 4-wave workgroups pair up per CU, and in a
 // sparse last round run alone at higher speed.  8 waves halve the streamed
@@ -519,6 +520,21 @@ int attn_waves(int B, int H, int S) {
     const int64_t wg = (int64_t)B * H * ((S + 255) / 256);
     const int64_t last = wg % n == 0 ? n : wg % n;
     return 2 * last >= n ? 8 : 4;
+}
+
+// The forward also takes 4 waves past the first round (two workgroups per CU)
+// where the last round of that grid gives no CU more than one: each then has
+// its CU to itself, while the 8-wave grid runs a half-empty round at full
+// length.  D = 128, us for 8 / 4 waves: B2 H24 S2048 120 / 104, B1 H24 S4096
+// 217 / 193, B4 H24 S1024 70 / 60, B6 H24 S600 58 / 48, B4 H20 S2048 190 / 164,
+// B2 H28 S4096 438 / 417; D = 64: S4096 145 / 123, B6 H24 S600 37 / 31.  With
+// a few more workgroups: H26 S3840 210 / 212, H25 S4096 215 / 224, B3 H24 S1400
+// 91 / 90.  (The backward's pair grid and its stored dS measure the same there:
+// B2 S2048 347 / 349.)
+static int fwd_waves(int B, int H, int S) {
+    const int nw = attn_waves(B, H, S), n = device_cu_count();
+    const int64_t wg = (int64_t)B * H * ((S + 127) / 128), last = wg % (2 * n);
+    return nw == 8 && wg > 2 * n && last > 0 && last <= n ? 4 : nw;
 }
 
 // Range split for grids that leave most CUs idle: with at most half the CUs
@@ -577,7 +593,7 @@ hipError_t launch_attn_fwd_bf16(const AttnFwdParams &p, int D, hipStream_t s) {
             hipLaunchKernelGGL(attn_fwd_combine_kernel<64>, cgrid, cblock, 0, s, p);
         return hipGetLastError();
     }
-    const int nw = attn_waves(p.B, p.H, p.S);
+    const int nw = fwd_waves(p.B, p.H, p.S);
     const int bm = nw * 32;
     const int nq = (p.S + bm - 1) / bm;
     const dim3 grid(p.B * p.H * nq), block(nw * 64);
