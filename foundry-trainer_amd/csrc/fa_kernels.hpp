@@ -48,7 +48,8 @@ struct AttnBwdParams {
     // ([split][B*H*S][D] per gradient) here and a reduce pass writes dq, dk, dv.
     int split;
     float *part_dq, *part_dk, *part_dv;
-    // dS through the workspace (ds != nullptr, unsplit bf16 only): dK/dV also
+    // dS through the workspace (ds != nullptr; unsplit bf16, and f32 in its
+    // own block layout, see attn_f32.hip): dK/dV also
     // stores the unscaled bf16 dS^T = (P * (dP - delta))^T of every (key,
     // query) as [B*H][S keys][ds_ld queries], and dQ = scale * dS K is a
     // streaming product over it instead of recomputing S and dP.
@@ -61,9 +62,9 @@ hipError_t launch_attn_fwd_bf16(const AttnFwdParams &p, int D, hipStream_t s);
 hipError_t launch_attn_fwd_f32(const AttnFwdParams &p, int D, hipStream_t s);
 // phase: 0 all, 1 pre-pass, 2 dK/dV, 3 dQ
 hipError_t launch_attn_bwd_bf16(const AttnBwdParams &p, int D, int phase, hipStream_t s);
-// Waves per workgroup (4 or 8, i.e. 128- or 256-row tiles) of the bf16
-// forward and the D = 128 backward kernels for B x H sequences of S tokens on
-// the current device (see attn_fwd.hip), when they run unsplit.
+// Waves per workgroup (4 or 8, i.e. 128- or 256-row tiles) of the D = 128 bf16
+// backward kernels for B x H sequences of S tokens on the current device, when
+// they run unsplit; the forward's but for fwd_waves (see attn_fwd.hip).
 int attn_waves(int B, int H, int S);
 // Range split factor (1 = none) of the bf16 kernels for B x H sequences of S
 // tokens on the current device: > 1 when even 8-wave workgroups would leave
