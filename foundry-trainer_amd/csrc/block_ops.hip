@@ -13,8 +13,11 @@
 // f32, results are rounded once to the storage type.
 #include <math.h>
 
+#include <type_traits>
+
 #include "fa_device.hpp"
 #include "fa_kernels.hpp"
+#include "fa_lds.hpp"
 
 namespace fa {
 namespace {
@@ -163,74 +166,110 @@ __global__ __launch_bounds__(256) void ln_mod_fwd_kernel(LnModParams p) {
     }
 }
 
-// Backward: a row is spread over W = ceil(C / 512) waves, lane l of wave w
-// holding elements w*512 + 8*l .. +8 in one 16-byte access per operand (two
-// for f32); a workgroup (block (64 W, R)) holds R rows, W R <= 8 waves.  With
-// one element group per lane all of a row's operands, the residual's gradient
-// and the gate among them, load at once in few registers: 30 waves share a CU.
-// Against a wave per row (six groups a lane, the residual loaded after the
-// sums, 4 waves per SIMD: 4608 rows are 1.1 rounds) 4608 x 3072 bf16 from cold
-// HBM 33 -> 27 us.  The forward keeps a wave per row: with one operand a row,
-// spread rows leave too few bytes in flight per CU (12 against 16 us).
+// 8 consecutive elements as they lie in memory, at byte offset off of a row's
+// buffer descriptor: past its end they read as zero.
+struct RawBf16 {
+    u32x4 w;
+};
+struct RawF32 {
+    u32x4 w, w2;
+};
+__device__ __forceinline__ void load_raw(__amdgpu_buffer_rsrc_t rs, int e, RawBf16 &r) {
+    r.w = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, e * 2, 0, 0));
+}
+__device__ __forceinline__ void load_raw(__amdgpu_buffer_rsrc_t rs, int e, RawF32 &r) {
+    r.w = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, e * 4, 0, 0));
+    r.w2 = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, e * 4 + 16, 0, 0));
+}
+__device__ __forceinline__ float raw_at(const RawBf16 &r, int j) { return (float)as_bf16x8(r.w)[j]; }
+__device__ __forceinline__ float raw_at(const RawF32 &r, int j) {
+    return j < 4 ? __builtin_bit_cast(f32x4, r.w)[j] : __builtin_bit_cast(f32x4, r.w2)[j - 4];
+}
+// Keeps r as it is (the compiler may not carry values derived from it across).
+__device__ __forceinline__ void raw_keep(RawBf16 &r) { asm volatile("" : "+v"(r.w)); }
+__device__ __forceinline__ void raw_keep(RawF32 &r) { asm volatile("" : "+v"(r.w), "+v"(r.w2)); }
+
+// Backward, one wave (and workgroup) per row: lane l holds elements
+// k*512 + 8*l .. +8 for k < MAXCH and sums them in that order, then the wave
+// its lanes, so a row's bits depend on no launch shape.
+//
+// HBM-bound.  All of a row's operands, the residual's gradient among them, are
+// loaded before any is used and stay in storage form (x and dy are widened
+// again after the sums): five waves per SIMD hold a 4608-row grid in one
+// round.  4608 x 3072 bf16 from cold HBM 31.1 -> 27.2 us (5.3 TB/s), with
+// GATE_OUT 38.9 -> 32.0, against loads chunk by chunk as the sums need them.
+// A row spread over six waves took 25.2 and 30.0, but adds in another order:
+// dx then differs in bf16 roundings.
 //
 // GATE_OUT: also gdx = g * dx, from dx as rounded to T (the same fma as the
 // gated-residual op with no x), the gradient through a gated branch whose
 // output fed this layer norm's input.
-template <typename T, bool GATE_OUT>
-__global__ __launch_bounds__(512) void ln_mod_bwd_kernel(LnModParams p) {
-    __shared__ float red[2][8];
-    const int64_t row = (int64_t)blockIdx.x * blockDim.y + threadIdx.y;
-    const int C = p.C, e = threadIdx.x * 8;
-    const bool in = row < p.N && e < C;  // lanes past the row (or the rows) still meet the others at the barrier
-    float n[8], dn[8], r[8], gv[8];
-    float a = 0.f, b = 0.f, rstd = 0.f;
+template <typename T, int MAXCH, bool GATE_OUT>
+__global__ __launch_bounds__(64) void ln_mod_bwd_kernel(LnModParams p) {
+    // each product and sum below rounds by itself, but for the fmas written out
+#pragma clang fp contract(off)
+    using Raw = std::conditional_t<sizeof(T) == 2, RawBf16, RawF32>;
+    const int lane = threadIdx.x;
+    const int64_t row = blockIdx.x;
+    const int C = p.C;
+    const uint32_t bytes = (uint32_t)C * sizeof(T);
+    const T *dres = static_cast<const T *>(p.dres);
+    const __amdgpu_buffer_rsrc_t xrs = make_rsrc(static_cast<const T *>(p.x) + row * p.ldx, bytes);
+    const __amdgpu_buffer_rsrc_t yrs = make_rsrc(static_cast<const T *>(p.dy) + row * p.lddy, bytes);
+    const __amdgpu_buffer_rsrc_t rrs = make_rsrc(dres ? dres + row * p.ldres : dres, dres ? bytes : 0u);
+    const __amdgpu_buffer_rsrc_t srs = make_rsrc(p.scale, bytes), grs = make_rsrc(p.g, bytes);
+    Raw x[MAXCH], dy[MAXCH], res[MAXCH], sc, sc1;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) n[j] = dn[j] = r[j] = gv[j] = 0.f;
-    if (in) {
-        float xv[8], dyv[8], sc[8];
-        load8(static_cast<const T *>(p.x) + row * p.ldx + e, xv);
-        load8(static_cast<const T *>(p.dy) + row * p.lddy + e, dyv);
-        if (p.dres) load8(static_cast<const T *>(p.dres) + row * p.ldres + e, r);
-        load8(static_cast<const T *>(p.scale) + e, sc);
-        if constexpr (GATE_OUT) load8(static_cast<const T *>(p.g) + e, gv);
-        const float mean = p.mean[row];
-        rstd = p.rstd[row];
+    for (int k = 0; k < MAXCH; ++k) {
+        load_raw(xrs, k * 512 + lane * 8, x[k]);
+        load_raw(yrs, k * 512 + lane * 8, dy[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < MAXCH; ++k) load_raw(rrs, k * 512 + lane * 8, res[k]);
+    load_raw(srs, lane * 8, sc);
+    __builtin_amdgcn_sched_barrier(0);  // the compiler would move most of them down to their uses
+    const float mean = p.mean[row], rstd = p.rstd[row];
+    float a = 0.f, b = 0.f;
+    // elements past C have dy = 0 and change neither sum
+#pragma unroll
+    for (int k = 0; k < MAXCH; ++k) {
+        load_raw(srs, (k + 1) % MAXCH * 512 + lane * 8, sc1);  // at last chunk 0's again, for the results
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            n[j] = (xv[j] - mean) * rstd;
-            dn[j] = dyv[j] * (sc[j] + 1.f);
-            a += dn[j];
-            b += dn[j] * n[j];
+            const float g = raw_at(sc, j) + 1.f, d = raw_at(dy[k], j);
+            const float n = (raw_at(x[k], j) - mean) * rstd;
+            a = __builtin_fmaf(g, d, a);
+            b = __builtin_fmaf(g * d, n, b);
         }
+        sc = sc1;
+        __builtin_amdgcn_sched_barrier(0);
     }
-    // both sums share one barrier
-    const int W = blockDim.x >> 6, base = threadIdx.y * W;
-    a = wave_sum(a);
-    b = wave_sum(b);
-    if (W > 1) {
-        if ((threadIdx.x & 63) == 0) {
-            red[0][base + (threadIdx.x >> 6)] = a;
-            red[1][base + (threadIdx.x >> 6)] = b;
-        }
-        __syncthreads();
-        a = red[0][base];
-        b = red[1][base];
-        for (int w = 1; w < W; ++w) {
-            a += red[0][base + w];
-            b += red[1][base + w];
-        }
-    }
-    if (!in) return;
-    const float ma = a / (float)C, mb = b / (float)C;
-    float o[8];
+    const float ma = wave_sum(a) / (float)C, mb = wave_sum(b) / (float)C;
+    Raw gt;
+    if constexpr (GATE_OUT) load_raw(grs, lane * 8, gt);
+    T *dx = static_cast<T *>(p.dx) + row * p.lddx, *gdx = static_cast<T *>(p.gdx) + row * p.ldgdx;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = r[j] + rstd * (dn[j] - ma - n[j] * mb);
-    store8(static_cast<T *>(p.dx) + row * p.lddx + e, o);
-    if constexpr (GATE_OUT) {
-        float go[8];
+    for (int k = 0; k < MAXCH; ++k) {
+        raw_keep(x[k]);
+        raw_keep(dy[k]);
+        float o[8], go[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) go[j] = __builtin_fmaf(gv[j], round_to<T>(o[j]), 0.f);
-        store8(static_cast<T *>(p.gdx) + row * p.ldgdx + e, go);
+        for (int j = 0; j < 8; ++j) {
+            const float n = (raw_at(x[k], j) - mean) * rstd, dn = (raw_at(sc, j) + 1.f) * raw_at(dy[k], j);
+            o[j] = __builtin_fmaf(rstd, __builtin_fmaf(-mb, n, dn - ma), raw_at(res[k], j));
+            if constexpr (GATE_OUT) go[j] = __builtin_fmaf(raw_at(gt, j), round_to<T>(o[j]), 0.f);
+        }
+        // the next vectors before this chunk's stores: the wait for them then leaves the stores in flight
+        __builtin_amdgcn_sched_barrier(0);
+        if (k + 1 < MAXCH) {
+            load_raw(srs, (k + 1) * 512 + lane * 8, sc);
+            if constexpr (GATE_OUT) load_raw(grs, (k + 1) * 512 + lane * 8, gt);
+        }
+        if (lane * 8 < C - k * 512) {
+            store8(dx + k * 512 + lane * 8, o);
+            if constexpr (GATE_OUT) store8(gdx + k * 512 + lane * 8, go);
+        }
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -423,9 +462,13 @@ static hipError_t ln_fwd_t(const LnModParams &p, hipStream_t s) {
 }
 template <typename T, bool F>
 static hipError_t ln_bwd_t(const LnModParams &p, hipStream_t s) {
-    const int W = (p.C + 511) / 512, R = 8 / W;  // waves per row (C <= 4096), rows per workgroup
-    const dim3 grid((unsigned)((p.N + R - 1) / R)), block(64 * W, R);
-    hipLaunchKernelGGL((ln_mod_bwd_kernel<T, F>), grid, block, 0, s, p);
+    const dim3 grid((unsigned)p.N), block(64);
+    if (p.C <= 1024)
+        hipLaunchKernelGGL((ln_mod_bwd_kernel<T, 2, F>), grid, block, 0, s, p);
+    else if (p.C <= 3072)
+        hipLaunchKernelGGL((ln_mod_bwd_kernel<T, 6, F>), grid, block, 0, s, p);
+    else
+        hipLaunchKernelGGL((ln_mod_bwd_kernel<T, 8, F>), grid, block, 0, s, p);
     return hipGetLastError();
 }
 template <typename T>

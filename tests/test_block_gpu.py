@@ -112,6 +112,56 @@ def test_fused_gated_ln_mod_matches_separate_ops(dtype, C):
     assert bool((gwide[:, C:] == 7.0).all()), "gated_out wrote past its view"
 
 
+def _wave_sum(s):
+    """The kernels' sum over a wave's 64 lanes (last axis), in f32."""
+    lane = torch.arange(64)
+    for partner in (lane ^ 1, lane ^ 2, lane ^ 7, lane ^ 15, lane ^ 16, lane ^ 32):
+        s = s + s[..., partner]
+    return s[..., 0]
+
+
+def _fma(a, b, c):
+    return (a.double() * b.double() + c.double()).float()
+
+
+@pytest.mark.parametrize("dres", [True, False])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,C", [(301, 8), (301, 256), (37, 520), (301, 768), (301, 1536), (66, 2048), (301, 3072),
+                                 (5, 3080), (301, 4096)])
+def test_ln_mod_bwd_sums_in_a_fixed_order(N, C, dtype, dres):
+    """dx is what one order of the row sums gives, bit for bit, at every width:
+    lane l adds elements 512 k + 8 l .. +8 for k = 0, 1, ..., then the lanes
+    meet pairwise.  Emulated here with each fma as one f64 product and sum."""
+    gen = torch.Generator().manual_seed(N * 8192 + C)
+    x, dy, r = (torch.randn(N, C, generator=gen).to(dtype) for _ in range(3))
+    sc, sh, g = (0.1 * torch.randn(C, generator=gen).to(dtype) for _ in range(3))
+    cu = lambda t: t.to("cuda")
+    _, mean, rstd = fb.ln_mod_fwd(cu(x), cu(sh), cu(sc), 1e-6, stats=True)
+    res = cu(r) if dres else None
+    dx = fb.ln_mod_bwd(cu(x), cu(dy), cu(sc), mean, rstd, 1e-6, dres=res)
+    dxg, gdx = fb.ln_mod_bwd_gate(cu(x), cu(dy), cu(sc), mean, rstd, cu(g), 1e-6, dres=res)
+    in_place = cu(dy)
+    fb.ln_mod_bwd(cu(x), in_place, cu(sc), mean, rstd, 1e-6, dres=res, out=in_place)
+    torch.cuda.synchronize()
+
+    m, rs = mean.cpu()[:, None], rstd.cpu()[:, None]
+    n, one_sc = (x.float() - m) * rs, sc.float() + 1
+    dn = dy.float() * one_sc
+    W = (C + 511) // 512
+    lanes = lambda t: torch.nn.functional.pad(t.expand(N, C), (0, 512 * W - C)).reshape(N, W, 64, 8)
+    d_l, s_l, n_l, dn_l = lanes(dy.float()), lanes(one_sc), lanes(n), lanes(dn)
+    a = b = torch.zeros(N, 64)
+    for k in range(W):
+        for j in range(8):
+            a = _fma(s_l[:, k, :, j], d_l[:, k, :, j], a)
+            b = _fma(dn_l[:, k, :, j], n_l[:, k, :, j], b)
+    ma, mb = (_wave_sum(t)[:, None] / torch.tensor(float(C)) for t in (a, b))
+    want = _fma(rs, _fma(-mb, n, dn - ma), r.float() if dres else torch.zeros(())).to(dtype)
+    for name, got in (("dx", dx), ("dx beside gdx", dxg), ("dx in place", in_place)):
+        assert torch.equal(got.cpu(), want), (name, int((got.cpu() != want).sum()))
+    assert torch.equal(gdx.cpu(), (g.float() * want.float()).to(dtype))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_swiglu_fused_views_match_oracle(dtype):
     """silu(gate) * up and its gradients with gate and up read as column
