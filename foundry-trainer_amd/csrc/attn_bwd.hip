@@ -241,9 +241,7 @@ __device__ __forceinline__ void dkdv_block(const AttnBwdParams &p, int work) {
         if (!live) {
             const u32x4 z = {0u, 0u, 0u, 0u};
             for (int blk = 0; blk < p.ds_ld / 16; ++blk) {
-                __builtin_amdgcn_raw_buffer_store_b128(z, dsrs, (uint32_t)lane * 16, (ds_row + (uint32_t)blk) * 1024,
-                                                       kDsCachePolicy);
-                asm volatile("s_nop 1" ::"v"(z));  // see the stores below
+                buffer_store_16<kDsCachePolicy>(z, dsrs, (uint32_t)lane * 16, (ds_row + (uint32_t)blk) * 1024);
             }
         }
     }
@@ -316,16 +314,8 @@ __device__ __forceinline__ void dkdv_block(const AttnBwdParams &p, int work) {
                     const auto r1 = __builtin_amdgcn_permlane32_swap(u[1], u[3], false, false);
                     u32x4 w = u32x4{r0[0], r1[0], r0[1], r1[1]};
                     if (ds_zero && !dkeep) w = u32x4{0u, 0u, 0u, 0u};
-                    __builtin_amdgcn_raw_buffer_store_b128(w, dsrs, (uint32_t)lane * 16,
-                                                           (ds_row + (uint32_t)(qb * 4 + sub * 2 + j)) * 1024,
-                                                           kDsCachePolicy);
-                    // A VALU write to a data VGPR of a 16-byte store in the
-                    // next cycle corrupted the stored first dword (measured:
-                    // every dword 0 of the blocks, nondeterministically; the
-                    // compiler emitted the write right after the store).
-                    // Holding the data live across wait states keeps the
-                    // write back.
-                    asm volatile("s_nop 1" ::"v"(w));
+                    buffer_store_16<kDsCachePolicy>(w, dsrs, (uint32_t)lane * 16,
+                                                    (ds_row + (uint32_t)(qb * 4 + sub * 2 + j)) * 1024);
                 }
             }
         }

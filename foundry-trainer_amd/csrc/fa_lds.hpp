@@ -124,6 +124,29 @@ __device__ __forceinline__ void buffer_to_lds_4(__amdgpu_buffer_rsrc_t rsrc, cha
                                              voff, soff, 0, 0);
 }
 
+// 16 bytes per lane and element of v to rsrc at (voff + soff + i * step),
+// POLICY the cache policy; bytes past the descriptor's range are dropped.  The
+// one 16-byte buffer store of this library: a VALU write to a data VGPR in the
+// instruction after such a store with its offset in an SGPR corrupted the
+// first stored dword, on some runs (the compiler holds no wait states for that
+// form).  All data stay live across an s_nop after the last store, so that
+// their registers are written two wait states later at the earliest.
+template <int POLICY, int N>
+__device__ __forceinline__ void buffer_store_16(const u32x4 (&v)[N], __amdgpu_buffer_rsrc_t rsrc, uint32_t voff,
+                                                uint32_t soff, uint32_t step) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+        __builtin_amdgcn_raw_buffer_store_b128(v[i], rsrc, voff, soff + (uint32_t)i * step, POLICY);
+    asm volatile("s_nop 1" ::"v"(v[0]));
+#pragma unroll
+    for (int i = 1; i < N; ++i) asm volatile("" ::"v"(v[i]));
+}
+template <int POLICY>
+__device__ __forceinline__ void buffer_store_16(u32x4 v, __amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff) {
+    const u32x4 one[1] = {v};
+    buffer_store_16<POLICY>(one, rsrc, voff, soff, 0u);
+}
+
 // Workgroup barrier that keeps buffer->LDS loads in flight.  __syncthreads()
 // drains every outstanding one (its workgroup release fence counts them as
 // pending LDS writes), which would cap a prefetch at one stage.  Here each

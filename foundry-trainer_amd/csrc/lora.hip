@@ -156,9 +156,10 @@ __global__ __launch_bounds__(256) void lora_expand_f32_kernel(const float *__res
     for (int j = 0; j < RP; ++j)
         w[j] = EXACT || j < R ? *reinterpret_cast<const f32x4 *>(wsh + j * LDW + lane * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
     for (int row = 0; row < rows; row += RB) {
-        f32x4 out[RB];
+        f32x4 prev[RB];
+        u32x4 out[RB];
 #pragma unroll
-        for (int i = 0; i < RB; ++i) out[i] = y[i];
+        for (int i = 0; i < RB; ++i) prev[i] = y[i];
         load(row + RB);
 #pragma unroll
         for (int i = 0; i < RB; ++i) {
@@ -171,9 +172,10 @@ __global__ __launch_bounds__(256) void lora_expand_f32_kernel(const float *__res
                 for (int e = 0; e < 4; ++e) acc[e] += uj * w[j][e];
             }
 #pragma unroll
-            for (int e = 0; e < 4; ++e) out[i][e] += s * acc[e];
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, out[i]), yrs, col * 4, (row + i) * yrow, 2);
+            for (int e = 0; e < 4; ++e) acc[e] = prev[i][e] + s * acc[e];
+            out[i] = __builtin_bit_cast(u32x4, acc);
         }
+        buffer_store_16<2>(out, yrs, col * 4, row * yrow, yrow);
     }
 }
 

@@ -40,3 +40,29 @@ def test_lora_f32_shapes(N, K, M, r, ypad, dxpad):
         err = float((got.double().cpu() - want).norm() / want.norm())
         assert err <= bound, (name, err, bound)
     assert torch.equal(yf[N].cpu().double(), y0[N]) and torch.equal(dxf[N].cpu().double(), dx0[N])
+
+
+@pytest.mark.parametrize("N,K,M,r", [(1536, 3072, 3072, 32), (1536, 3072, 3072, 16), (1025, 1024, 512, 32),
+                                     (257, 256, 260, 17), (37, 512, 256, 32), (5, 64, 128, 9), (1, 16, 16, 32)])
+def test_lora_f32_vector_up_products_by_element(N, K, M, r):
+    """y and dx with aligned rows, element by element: each within the rounding
+    of its own sums (N % 4 == 1 leaves a wave's last group of four rows with
+    one), and four rows past N untouched."""
+    torch.manual_seed(N + 7 * r)
+    x, dy = torch.randn(N, K, device="cuda"), torch.randn(N, M, device="cuda")
+    a, b = torch.randn(r, K, device="cuda"), torch.randn(M, r, device="cuda")
+    yf, dxf = torch.randn(N + 4, M, device="cuda"), torch.randn(N + 4, K, device="cuda")
+    y0, dx0 = yf.clone(), dxf.clone()
+    for _ in range(3):  # the same bits each time
+        yf.copy_(y0)
+        dxf.copy_(dx0)
+        u = lora_fwd(x, a, b, yf[:N], 0.5)
+        lora_bwd(x, a, b, u, dy, 0.5, dx=dxf[:N])
+        X, A, B, DY, Y0, DX0 = (t.double() for t in (x, a, b, dy, y0[:N], dx0[:N]))
+        for name, got, start, left, w1, w2, k in (("y", yf, Y0, X, A.t(), B.t(), K), ("dx", dxf, DX0, DY, B, A, M)):
+            want = start + 0.5 * left @ w1 @ w2
+            # k + r products and sums, the scale and the addition, each rounded to 2^-24
+            bound = 2.0 ** -24 * ((k + r + 3) * 0.5 * left.abs() @ w1.abs() @ w2.abs() + start.abs() + want.abs())
+            over = (got[:N].double() - want).abs() - bound
+            assert bool((over <= 0).all()), (name, int((over > 0).sum()), float(over.max()))
+        assert torch.equal(yf[N:], y0[N:]) and torch.equal(dxf[N:], dx0[N:])
