@@ -374,6 +374,15 @@ def _linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor], out: to
     return torch.addmm(b, x, w.t(), out=out)
 
 
+def _bwd_workspace(S: int, H: int, D: int, dtype, device) -> Optional[torch.Tensor]:
+    """The attention backward's workspace that a block keeps.  None for f32,
+    whose dS (4 H S^2 bytes: 2 GB at 4608 tokens and 24 heads, per block) is
+    attn_bwd's to allocate for the call, where there is room for it."""
+    if dtype == torch.float32:
+        return None
+    return torch.empty(attn_bwd_workspace_bytes(1, S, H, D, dtype), dtype=torch.uint8, device=device)
+
+
 class DoubleBlockLoRA:
     """One double-stream block with LoRA on q/k/v/out of both streams.
 
@@ -657,8 +666,7 @@ class DoubleBlockLoRA:
                  "o": torch.empty((1, S, H, D), **kw), "do": torch.empty((1, S, H, D), **kw),
                  "dq": torch.empty((1, S, H, D), **kw), "dk": torch.empty((1, S, H, D), **kw),
                  "lse": torch.empty((1, H, S), dtype=torch.float32, device=self.device),
-                 "ws": torch.empty(attn_bwd_workspace_bytes(1, S, H, D, self.dtype), dtype=torch.uint8,
-                                  device=self.device)}
+                 "ws": _bwd_workspace(S, H, D, self.dtype, self.device)}
             for name in STREAMS:
                 n = self.rows[name]
                 for key, width in (("h", C), ("out", C), ("x1", C), ("h2", C), ("y", C), ("t1", C),
@@ -1134,8 +1142,7 @@ class SingleBlockLoRA:
                 "q": torch.empty((1, S, H, D), **kw), "k": torch.empty((1, S, H, D), **kw),
                 "dq": torch.empty((1, S, H, D), **kw), "dk": torch.empty((1, S, H, D), **kw),
                 "lse": torch.empty((1, H, S), dtype=torch.float32, device=self.device),
-                "ws": torch.empty(attn_bwd_workspace_bytes(1, S, H, D, self.dtype), dtype=torch.uint8,
-                                  device=self.device)}
+                "ws": _bwd_workspace(S, H, D, self.dtype, self.device)}
             if self.fused:
                 P = ADAPTER_PAD
                 for key in ("nh_ext", "out_ext", "dout_ext", "dnh_ext"):  # padding columns stay zero

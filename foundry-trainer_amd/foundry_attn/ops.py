@@ -209,23 +209,25 @@ def attn_bwd(q, k, v, o, dout, lse, scale: Optional[float] = None, key_keep=None
     # a given workspace of at least the minimum is used as it is (below the
     # full size: dQ recomputes S and dP); none gets the full size (dQ reads
     # the dK/dV kernel's stored dS), or the minimum where memory has no room
-    # for the dS (up to FA_BWD_DS_MAX_BYTES): the same bits
+    # for the dS (up to FA_BWD_DS_MAX_BYTES): the same bits.  f32 takes the
+    # minimum too where its dS would not be used (separate phases) or would
+    # stay in a captured graph's memory for the graph's life
     given = 0 if workspace is None else workspace.numel() * workspace.element_size()
+    size = lambda which: _abi.entry(f"fa_attn_bwd_{which}_workspace_size", size=True)(_pack_bwd(*head, 0, 0, *strides))
     least = 0
     if workspace is not None:
-        least = _abi.entry("fa_attn_bwd_min_workspace_size", size=True)(_pack_bwd(*head, 0, 0, *strides))
+        least = size("min")
     if workspace is None or given < least:
         if workspace is not None and phases is not None:
             # separate phase calls share the pre-pass rows through it
             raise FoundryAttnError(_abi.FA_ERR_INVALID_ARG,
                                    f"workspace of {given} bytes is smaller than the {least} these shapes need")
-        need = _abi.entry("fa_attn_bwd_ds_workspace_size", size=True)(_pack_bwd(*head, 0, 0, *strides))
-        given = max(need, 256)
+        rows_only = q4.dtype == torch.float32 and (phases is not None or torch.cuda.is_current_stream_capturing())
+        given = max(size("min" if rows_only else "ds"), 256)
         try:
             workspace = torch.empty(given, dtype=torch.uint8, device=q4.device)
         except torch.cuda.OutOfMemoryError:
-            least = least or _abi.entry("fa_attn_bwd_min_workspace_size", size=True)(_pack_bwd(*head, 0, 0, *strides))
-            given = max(least, 256)
+            given = max(size("min"), 256)
             workspace = torch.empty(given, dtype=torch.uint8, device=q4.device)
     args = _pack_bwd(*head, workspace.data_ptr(), given, *strides)
     if phases is None:

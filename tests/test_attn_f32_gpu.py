@@ -74,6 +74,42 @@ def test_backward_without_room_for_ds(monkeypatch, dtype, S, H):
         assert torch.equal(a, b)
 
 
+def test_graph_and_phases_hold_no_ds(monkeypatch):
+    """A captured f32 backward keeps no dS in its graph's memory, and separate
+    phases (which do not use it) allocate none: the same bits, on replays too."""
+    B, S, H, D = 1, 1056, 4, 128
+    ds_bytes = 4 * H * S * S
+    t = [torch.randn(B, S, H, D, device="cuda") for _ in range(4)]
+    out = [torch.empty_like(t[0]) for _ in range(3)]
+    o, lse = attn_fwd(*t[:3])
+    want = attn_bwd(*t[:3], o, t[3], lse)
+    sizes, empty = [], torch.empty
+
+    def recorded(*shape, **kw):
+        if kw.get("dtype") == torch.uint8:
+            sizes.append(shape[0])
+        return empty(*shape, **kw)
+
+    monkeypatch.setattr(torch, "empty", recorded)
+    phases = [(p, None) for p in (_abi.FA_BWD_PREPASS, _abi.FA_BWD_DKDV, _abi.FA_BWD_DQ)]
+    for a, b in zip(attn_bwd(*t[:3], o, t[3], lse, phases=phases), want):
+        assert torch.equal(a, b)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        attn_bwd(*t[:3], o, t[3], lse, out=out)
+    assert len(sizes) == 2 and max(sizes) < ds_bytes, sizes
+    for _ in range(3):
+        for g in out:
+            g.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(out, want):
+            assert torch.equal(a, b)
+    attn_bwd(*t[:3], o, t[3], lse)
+    assert sizes[-1] > ds_bytes  # the eager call still takes it
+
+
 @pytest.mark.parametrize("D", [64, 128])
 def test_row_stride_past_32_bit_offsets(D):
     """Rows 2^25 elements apart: a 32-row tile spans 4 GiB and more."""

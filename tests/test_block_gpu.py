@@ -13,6 +13,7 @@ import block_ref  # noqa: E402  (oracle/ on sys.path via conftest)
 import oracle
 from block_case import make_case, make_single_case, oracle_mods, single_oracle_mods
 from foundry_attn import block as fb
+from foundry_attn.ops import attn_bwd_workspace_bytes
 from helpers import check_gate, max_abs, rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -541,6 +542,19 @@ def device_single_block(case, dtype):
                              theta=case["theta"], lora_scale=case["scale"])
     blk.set_conditioning(dev(case["c"], dtype))
     return blk
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_blocks_keep_no_f32_ds(dtype):
+    """An f32 block keeps no workspace with room for dS (4 H S^2 bytes) beyond
+    its calls; a bf16 one keeps what its backward uses."""
+    bf = dtype == torch.bfloat16
+    double = device_block(make_case(C=256, H=2, T=40, rows=12, cols=12, r=4, bf16=bf), dtype)
+    single = device_single_block(make_single_case(C=256, H=2, T=40, rows=12, cols=12, r=4, bf16=bf), dtype)
+    for blk in (double, single):
+        kept = [t for t in blk._buffers().values() if t is not None and t.dtype == torch.uint8]
+        most = attn_bwd_workspace_bytes(1, blk.S, 2, 128, dtype, minimum=not bf)
+        assert sum(t.numel() for t in kept) <= most, (type(blk).__name__, [t.numel() for t in kept], most)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
