@@ -174,13 +174,10 @@ fa_status check_buffer_view(const char *name, const fa_strides &st, int32_t S, i
 
 size_t round256(size_t x) { return (x + 255) & ~size_t(255); }
 
-// Range split factor the workspaces hold room for (1 for f32 or shapes that
-// never split), and the one a call runs with.
+// Range split factor a call runs with, and its workspaces hold room for: 1 for
+// f32, and where a split would not pay.
 int split_for(int32_t dtype, int32_t B, int32_t S, int32_t H) {
-    return dtype == FA_DTYPE_BF16 ? fa::attn_split(B, H, S) : 1;
-}
-int split_used(int32_t dtype, int32_t B, int32_t S, int32_t H) {
-    const int split = split_for(dtype, B, S, H);
+    const int split = dtype == FA_DTYPE_BF16 ? fa::attn_split(B, H, S) : 1;
     return fa::attn_split_pays(S, split) ? split : 1;
 }
 
@@ -203,35 +200,33 @@ size_t bwd_min_workspace(int32_t dtype, int32_t B, int32_t S, int32_t H, int32_t
 // are 32-bit).
 // Past FA_BWD_DS_MAX_BYTES of dS (16 GiB) a call keeps the recomputing path
 // rather than ask for a workspace of that size.
+//
+// bf16 dS pays at D = 128 only: at D = 64 its traffic is the same for half the
+// products saved, and the 4-wave recomputing kernels are faster (B1 H24 S4608
+// D64: 562 us through dS, 471 recomputing).
 int ds_ld_for(int32_t S) { return (S + 255) / 256 * 256; }
-size_t bwd_ds_bytes(int32_t dtype, int32_t B, int32_t S, int32_t H) {
+size_t bwd_ds_bytes(int32_t dtype, int32_t B, int32_t S, int32_t H, int32_t D) {
     if (dtype == FA_DTYPE_F32) {
         if (S > (1 << 22)) return 0;  // as the call itself; keeps the products below in 64 bits
         const size_t nb = (size_t)(S + 31) / 32;
         const size_t head = nb * nb * 4096, heads = (size_t)B * (size_t)H;
         return heads > (size_t)FA_BWD_DS_MAX_BYTES / head ? 0 : heads * head;
     }
-    if (dtype != FA_DTYPE_BF16 || split_for(dtype, B, S, H) > 1 || fa::attn_waves(B, H, S) != 8) return 0;
+    if (dtype != FA_DTYPE_BF16 || D != 128 || split_for(dtype, B, S, H) > 1 || fa::attn_waves(B, H, S) != 8) return 0;
     const int64_t head = (int64_t)(S + 31) / 32 * 32 * ds_ld_for(S) * 2;
     if (head >= (int64_t(1) << 32)) return 0;
     const size_t bytes = round256((size_t)B * H * head);
     return bytes > (size_t)FA_BWD_DS_MAX_BYTES ? 0 : bytes;
 }
 
-// bf16 dS pays at D = 128 only: at D = 64 its traffic is the same for half the
-// products saved, and the 4-wave recomputing kernels are faster (B1 H24 S4608
-// D64: 562 us through dS, 471 recomputing).
-bool stores_ds(int32_t dtype, int32_t D) { return dtype == FA_DTYPE_F32 || D == 128; }
-
 size_t bwd_ds_workspace(int32_t dtype, int32_t B, int32_t S, int32_t H, int32_t D) {
-    return bwd_min_workspace(dtype, B, S, H, D) + (stores_ds(dtype, D) ? bwd_ds_bytes(dtype, B, S, H) : 0);
+    return bwd_min_workspace(dtype, B, S, H, D) + bwd_ds_bytes(dtype, B, S, H, D);
 }
 
 // What a caller that asks no further is told: f32 calls keep their rows only
-// (their dS is twice bf16's size), bf16 ones get room for dS, at D = 64 too
-// (a size callers may have fixed; those calls leave it unused).
+// (their dS is twice bf16's size).
 size_t bwd_workspace(int32_t dtype, int32_t B, int32_t S, int32_t H, int32_t D) {
-    return bwd_min_workspace(dtype, B, S, H, D) + (dtype == FA_DTYPE_F32 ? 0 : bwd_ds_bytes(dtype, B, S, H));
+    return dtype == FA_DTYPE_F32 ? bwd_min_workspace(dtype, B, S, H, D) : bwd_ds_workspace(dtype, B, S, H, D);
 }
 
 // forward workspace of a split call: O partials [split][B,H,S][D] f32, then
@@ -310,7 +305,7 @@ fa_status fa_attn_fwd(const fa_attn_fwd_args *a, void *stream) {
                         "workspace of %zu bytes is smaller than the %zu a split forward needs (NULL runs unsplit)",
                         a->workspace_bytes, need);
         if (need > 0) {
-            p.split = split_used(a->dtype, a->batch, a->seq, a->heads);
+            p.split = split_for(a->dtype, a->batch, a->seq, a->heads);
             p.part_o = static_cast<float *>(a->workspace);
             p.part_lse = reinterpret_cast<float *>(
                 static_cast<char *>(a->workspace) +
@@ -417,7 +412,7 @@ fa_status fa_attn_bwd_phase(const fa_attn_bwd_args *a, int32_t phase, void *stre
         return fail(FA_ERR_INVALID_ARG, "unknown backward phase %d", phase);
     FA_TRY(check_bwd_args(a));
     const size_t need = bwd_min_workspace(a->dtype, a->batch, a->seq, a->heads, a->head_dim);
-    const size_t ds = bwd_ds_bytes(a->dtype, a->batch, a->seq, a->heads);
+    const size_t ds = bwd_ds_bytes(a->dtype, a->batch, a->seq, a->heads, a->head_dim);
     if (!a->workspace || !aligned(a->workspace, 256))
         return fail(FA_ERR_INVALID_ARG, "workspace is NULL or not 256-byte aligned");
     if (a->workspace_bytes < need)
@@ -426,8 +421,8 @@ fa_status fa_attn_bwd_phase(const fa_attn_bwd_args *a, int32_t phase, void *stre
     FA_TRY(init_current());
 
     fa::AttnBwdParams p;
-    fill_bwd_params(a, static_cast<char *>(a->workspace), split_used(a->dtype, a->batch, a->seq, a->heads),
-                    ds > 0 && a->workspace_bytes >= need + ds && stores_ds(a->dtype, a->head_dim), p);
+    fill_bwd_params(a, static_cast<char *>(a->workspace), split_for(a->dtype, a->batch, a->seq, a->heads),
+                    ds > 0 && a->workspace_bytes >= need + ds, p);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const hipError_t e = a->dtype != FA_DTYPE_BF16 ? fa::launch_attn_bwd_f32(p, a->head_dim, phase, s)
                                                    : fa::launch_attn_bwd_bf16(p, a->head_dim, phase, s);

@@ -107,7 +107,7 @@ def attn_fwd(q, k, v, scale: Optional[float] = None, key_keep=None, out=None, ls
     to 1/sqrt(D) (the reference hard-codes 1/sqrt(128), lib.rs:138).
     key_keep: optional (B,S) bool/uint8 mask, False = key excluded.
     split: pass a workspace so that a grid too small for the GPU (few heads,
-    fa_attn_fwd_workspace_size > 0) may split each tile's keys; `workspace` is
+    fa_attn_fwd_workspace_size > 0) splits each tile's keys; `workspace` is
     used when large enough, else one is allocated.  split=False runs the
     unsplit kernel.
     Returns o (same shape as q) and lse (B,H,S) float32.

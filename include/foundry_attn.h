@@ -102,19 +102,19 @@ typedef struct fa_attn_fwd_args {
 
 /* Bytes of workspace a split forward needs for these shapes: nonzero for bf16
  * when B x H x ceil(S/256) workgroups would leave at least half of the
- * current device's CUs idle and S >= 1024 (for example 3 or 6 heads at
- * S = 4608: one GPU's share of 24 heads over 8 or 4 GPUs).  Each query tile's
- * keys may then be cut into up to 16 ranges of >= 512 keys on separate
- * workgroups, whose f32 partials are merged through their LSEs (where that is
- * faster: three ranges or more, or two from seq 4608 on).  0 means the forward
- * never splits these shapes.  No reference counterpart. */
+ * current device's CUs idle, S >= 1024 (for example 3 or 6 heads at
+ * S = 4608: one GPU's share of 24 heads over 8 or 4 GPUs) and splitting is the
+ * faster: into three ranges or more, or two from seq 4608 on.  Each query
+ * tile's keys are then cut into up to 16 ranges of >= 512 keys on separate
+ * workgroups, whose f32 partials are merged through their LSEs.  0 means the
+ * forward never splits these shapes.  No reference counterpart. */
 size_t fa_attn_fwd_workspace_size(const fa_attn_fwd_args *args);
 
 /* O = softmax(Q K^T * scale) V per (b, h), scores and softmax in f32, P cast to
  * the storage dtype before P V (lib.rs:131-149), plus the per-row LSE that the
  * backward uses to recompute P.  A fully masked row gives O = 0, LSE = -inf.
  * With workspace NULL the call never splits; with a workspace of at least
- * fa_attn_fwd_workspace_size bytes it may split the shapes that size covers (a
+ * fa_attn_fwd_workspace_size bytes it splits the shapes that size covers (a
  * smaller non-NULL workspace is FA_ERR_INVALID_ARG).  Results are
  * deterministic either way.  Replaces AttnBwd::cuda_fwd (lib.rs:189-214) and
  * AttnBwd::cpu_fwd (lib.rs:158-187). */
@@ -139,28 +139,29 @@ typedef struct fa_attn_bwd_args {
  * pre-pass rows, plus, for the shapes fa_attn_fwd_workspace_size splits, f32
  * partial sums of dQ, dK and dV (dQ's key range and dK/dV's query range are
  * split the same way, and a reduce pass adds the partials in a fixed order),
- * plus, for unsplit bf16 calls with 8-wave workgroups, the bf16 dS of every
- * (key, query) pair ([B*H][seq rounded up to 32][seq rounded up to 256]),
- * through which dQ reads the dK/dV kernel's dS instead of recomputing S and
- * dP (about 1 GB at B1 H24 S4608; shapes whose dS would exceed
+ * plus, for unsplit bf16 calls with head_dim 128 and 8-wave workgroups, the
+ * bf16 dS of every (key, query) pair ([B*H][seq rounded up to 32][seq rounded
+ * up to 256]), through which dQ reads the dK/dV kernel's dS instead of
+ * recomputing S and dP (about 1 GB at B1 H24 S4608; shapes whose dS would exceed
  * FA_BWD_DS_MAX_BYTES keep the recomputing path and ask for no dS).  No
  * reference counterpart: AttnBwd::bwd (lib.rs:216-263) allocates its own
  * tensors. */
 #define FA_BWD_DS_MAX_BYTES (16ull << 30)
 size_t fa_attn_bwd_workspace_size(const fa_attn_bwd_args *args);
 
-/* The least workspace fa_attn_bwd accepts (0 on bad args): without the dS^T
- * rows, so dQ recomputes S and dP.  A workspace of at least
- * fa_attn_bwd_workspace_size bytes takes the stored-dS path, a smaller one
- * (of at least this size) the recomputing one.  Both multiply the same bf16
- * dS by K in the same key order, so they give the same bits.  No reference
- * counterpart. */
+/* The least workspace fa_attn_bwd accepts (0 on bad args): without the dS
+ * rows, so dQ recomputes S and dP.  Where fa_attn_bwd_ds_workspace_size is
+ * larger, a workspace of at least that many bytes takes the stored-dS path, a
+ * smaller one (of at least this size) the recomputing one.  Both multiply the
+ * same dS by K in the same key order, so they give the same bits.  No
+ * reference counterpart. */
 size_t fa_attn_bwd_min_workspace_size(const fa_attn_bwd_args *args);
 
 /* The workspace with which fa_attn_bwd stores dS wherever this build can (0 on
- * bad args): fa_attn_bwd_workspace_size for bf16; for f32 that plus the f32 dS
- * of every (key, query) pair ([B*H][seq][seq], both rounded up to 32; nothing
- * past FA_BWD_DS_MAX_BYTES of it).  An f32 fa_attn_bwd given this much forms
+ * bad args): fa_attn_bwd_workspace_size for bf16 (which at head_dim 64 stores
+ * none); for f32 that plus the f32 dS of every (key, query) pair
+ * ([B*H][seq][seq], both rounded up to 32; nothing past FA_BWD_DS_MAX_BYTES
+ * of it).  An f32 fa_attn_bwd given this much forms
  * dQ from the stored dS, with the bits of the recomputing dQ; less (down to
  * the minimum), the separate phases and fa_attn_bwd_noalloc recompute it, so
  * the f32 phases stay independent of each other with any workspace.  No
@@ -188,10 +189,10 @@ fa_status fa_attn_bwd(const fa_attn_bwd_args *args, void *stream);
  *   FA_BWD_DQ       dQ        (needs the pre-pass; through the stored dS,
  *                             also dK/dV, whose dS it reads)
  * FA_BWD_ALL runs all three, as fa_attn_bwd.  The caller orders the pre-pass
- * before the other two (same stream, or an event), and with a workspace of
- * fa_attn_bwd_workspace_size bytes (the stored-dS path, see above) dK/dV
- * before dQ; with fa_attn_bwd_min_workspace_size bytes dK/dV and dQ are
- * independent.  No reference counterpart: AttnBwd::bwd (lib.rs:216-263) is
+ * before the other two (same stream, or an event), and for bf16 with a
+ * workspace of fa_attn_bwd_workspace_size bytes (the stored-dS path, see
+ * above) dK/dV before dQ; with fa_attn_bwd_min_workspace_size bytes, and for
+ * f32, dK/dV and dQ are independent.  No reference counterpart: AttnBwd::bwd (lib.rs:216-263) is
  * one call. */
 typedef enum fa_bwd_phase {
     FA_BWD_ALL = 0,

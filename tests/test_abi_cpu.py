@@ -105,6 +105,22 @@ def test_fwd_validation_errors(field, value, code):
     assert len(lib().fa_last_error()) > 0
 
 
+def test_workspaces_of_grids_that_run_unsplit():
+    """Small grids whose split would not pay (two ranges below seq 4608) ask
+    for no split partials; three ranges, and two at seq 4608, do (256 CUs)."""
+    if gpu_available():
+        pytest.skip("sizes depend on the device's CUs; covered on 256 by the GPU tests")
+    for B, S, H, split in ((1, 1400, 2, 1), (1, 1024, 24, 1), (4, 3000, 2, 1), (1, 1600, 2, 3), (1, 4608, 6, 2)):
+        f = _abi.AttnFwdArgs(dtype=0, batch=B, seq=S, heads=H, head_dim=64)
+        b = _abi.AttnBwdArgs(dtype=0, batch=B, seq=S, heads=H, head_dim=64)
+        r256 = lambda n: (n + 255) // 256 * 256
+        rows, part = 2 * r256(B * H * S * 4), r256(split * B * H * S * 64 * 4) if split > 1 else 0
+        lse = r256(split * B * H * S * 4) if split > 1 else 0
+        assert lib().fa_attn_fwd_workspace_size(ctypes.byref(f)) == part + lse, (B, S, H)
+        for size in (lib().fa_attn_bwd_workspace_size, lib().fa_attn_bwd_min_workspace_size):
+            assert size(ctypes.byref(b)) == rows + 3 * part, (B, S, H)
+
+
 def test_null_args_pointer():
     assert lib().fa_attn_fwd(None, None) == _abi.FA_ERR_INVALID_ARG
     assert lib().fa_attn_bwd(None, None) == _abi.FA_ERR_INVALID_ARG
@@ -122,7 +138,7 @@ def test_bwd_workspace_size_and_validation():
     a.workspace, a.workspace_bytes = fake, need - 256
     assert lib().fa_attn_bwd(ctypes.byref(a), None) == _abi.FA_ERR_INVALID_ARG
     assert b"workspace" in lib().fa_last_error()
-    # 4-wave shapes and f32 have no stored-dS path: the full size is the least
+    # 4-wave shapes store no dS: the full size is the least
     assert lib().fa_attn_bwd_min_workspace_size(ctypes.byref(a)) == need
     # an 8-wave bf16 shape (44 heads x 5 tiles: 220 workgroups) adds the dS
     # blocks, [heads][S rounded up to 32][S rounded up to 256] bf16, and
@@ -136,6 +152,11 @@ def test_bwd_workspace_size_and_validation():
     b.dtype = 1
     assert lib().fa_attn_bwd_workspace_size(ctypes.byref(b)) == lib().fa_attn_bwd_min_workspace_size(ctypes.byref(b))
     b.dtype = 0
+    # D = 64 stores no dS: nothing is asked for it
+    d64 = _abi.AttnBwdArgs.from_buffer_copy(b)
+    d64.head_dim = 64
+    for size in (lib().fa_attn_bwd_workspace_size, lib().fa_attn_bwd_ds_workspace_size):
+        assert size(ctypes.byref(d64)) == lib().fa_attn_bwd_min_workspace_size(ctypes.byref(d64)) == least
     # past 16 GiB of dS (here 8 x 44 heads at S 8192: 47 GiB) no dS is asked for
     big = _abi.AttnBwdArgs.from_buffer_copy(b)
     big.batch, big.seq = 8, 8192

@@ -2,7 +2,8 @@
 GPU: one GPU's share of the heads under sequence parallelism).
 
 When B x H x ceil(S/256) workgroups would leave at least half of the CUs idle
-(S >= 1024), the forward and dQ cut each tile's keys, and dK/dV each tile's
+(S >= 1024), and the ranges would be three or more (or two from S = 4608 on),
+the forward and dQ cut each tile's keys, and dK/dV each tile's
 queries, into ranges run by separate workgroups; f32 partials are merged
 (forward: through their LSEs) or summed in a fixed order.  Gates as for the
 unsplit kernels: bf16 max-abs <= 2e-2 and rel-L2 <= 1e-2 against the CPU
@@ -58,8 +59,8 @@ def test_split_policy_and_workspace_sizes():
 
 
 @pytest.mark.parametrize("B,S,H,D,masked", [(1, 2048, 2, 128, False), (1, 2048, 2, 128, True),
-                                            (1, 1400, 2, 64, False), (2, 1500, 1, 128, True)],
-                         ids=["s2048", "s2048_masked", "s1400_d64", "b2_s1500_masked"])
+                                            (1, 1600, 2, 64, False), (2, 1500, 1, 128, True)],
+                         ids=["s2048", "s2048_masked", "s1600_d64", "b2_s1500_masked"])
 def test_split_parity_vs_oracle(B, S, H, D, masked):
     """Ragged and masked split shapes against the oracle on every head."""
     assert _splits(B, S, H, D)[0] > 0, "shape does not split"
@@ -172,12 +173,12 @@ def test_forward_workspace_too_small_is_refused():
 
 @pytest.mark.parametrize("seed", [1, 2, 3, 4, 5, 6])
 def test_split_random_shapes(seed):
-    """Seeded random split shapes (B 1-2, H 1-3, ragged S 1024-3000, D 64 or
+    """Seeded random split shapes (B 1-2, H 1-3, ragged S 1409-3000, D 64 or
     128, half of them with a random key mask that keeps every batch item's
     first key) against the oracle on one head."""
     rng = np.random.default_rng(100 + seed)
     B, H = int(rng.integers(1, 3)), int(rng.integers(1, 4))
-    S, D = int(rng.integers(1024, 3001)), int(rng.choice([64, 128]))
+    S, D = int(rng.integers(1409, 3001)), int(rng.choice([64, 128]))
     print(f"  B={B} S={S} H={H} D={D}", flush=True)
     assert _splits(B, S, H, D)[0] > 0, "shape does not split"
     from oracle import bf16_round
@@ -190,3 +191,24 @@ def test_split_random_shapes(seed):
     g = run_gpu(q, k, v, do, torch.bfloat16, scale, keep)
     h = int(rng.integers(0, H))
     compare(g, q, k, v, do, scale, keep, True, (h, h + 1))
+
+
+@pytest.mark.parametrize("B,S,H,D", [(1, 1400, 2, 64), (1, 1100, 4, 128), (4, 3000, 2, 128), (1, 1024, 24, 128)])
+def test_two_short_ranges_run_unsplit(B, S, H, D):
+    """Grids whose split would be in two, below S = 4608: no workspace beyond
+    the pre-pass rows is asked for, a workspace of the split's size is still
+    taken, and the bits are the unsplit kernels'."""
+    fwd, bwd = _splits(B, S, H, D)
+    assert fwd == 0 and bwd == 2 * ((B * H * S * 4 + 255) // 256 * 256)
+    torch.manual_seed(S)
+    q, k, v, do = (torch.randn(B, S, H, D, device="cuda").to(torch.bfloat16) for _ in range(4))
+    big = torch.empty(bwd + 3 * 2 * B * H * S * D * 4, dtype=torch.uint8, device="cuda")
+    o, lse = attn_fwd(q, k, v)
+    o2, lse2 = attn_fwd(q, k, v, workspace=big)
+    o3, lse3 = attn_fwd(q, k, v, split=False)
+    want = attn_bwd(q, k, v, o, do, lse)
+    got = attn_bwd(q, k, v, o, do, lse, workspace=big)
+    torch.cuda.synchronize()
+    assert torch.equal(o, o2) and torch.equal(lse, lse2) and torch.equal(o, o3) and torch.equal(lse, lse3)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
