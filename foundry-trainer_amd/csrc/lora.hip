@@ -199,7 +199,7 @@ __global__ __launch_bounds__(256) void lora_expand_f32_kernel(const float *__res
 // loop (the regions are private).  Rows >= N and j >= R load from a clamped (valid) row:
 // output element (n, j) depends on row n of X and row j of W only, and those
 // outputs are not stored.  A last k-step cut short by K (K is a multiple of
-// a 16-byte chunk) has its chunks past K zeroed in the X operand.
+// a 16-byte chunk) has its chunks past K zeroed in both operands.
 // One k-step per stage in bf16: two k-steps per stage (twice the LDS) was no
 // faster alone and slower in the c4 step, where a workgroup's LDS decides
 // whether it can share a CU with the other stream's kernels.  f32 rows have
@@ -277,18 +277,23 @@ __global__ __launch_bounds__(512) void lora_rowdot16_kernel(const T *__restrict_
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[mt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto consume = [&](int j0, const char *src) {
-        const char *d = src + wave * RS::WAVE;
+    auto consume = [&](int j0, char *src) {
+        char *d = src + wave * RS::WAVE;
 #pragma unroll
         for (int g = 0; g < G; ++g)
             if (j0 + g < J) {
+                // Columns past K, zeroed where they lie (this wave's own region):
+                // W's are the next row's first values, which may be infinite.
+                if (tail < 4 && wave + 8 * (j0 + g) == nks - 1 && q >= tail) {
+#pragma unroll
+                    for (int t = 0; t < MT + NT; ++t) *reinterpret_cast<u32x4 *>(d + g * RS::STEP + 1024 * t + rd) = zero;
+                }
                 u32x4 wf[NT];
 #pragma unroll
                 for (int t = 0; t < NT; ++t) wf[t] = ld_lds_16(d + g * RS::STEP + 1024 * (MT + t), rd);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
-                    u32x4 a = ld_lds_16(d + g * RS::STEP + 1024 * mt, rd);
-                    if (tail < 4 && wave + 8 * (j0 + g) == nks - 1 && q >= tail) a = zero;  // columns past K
+                    const u32x4 a = ld_lds_16(d + g * RS::STEP + 1024 * mt, rd);
 #pragma unroll
                     for (int t = 0; t < NT; ++t) {
                         if constexpr (E == 2) {

@@ -66,3 +66,27 @@ def test_lora_f32_vector_up_products_by_element(N, K, M, r):
             over = (got[:N].double() - want).abs() - bound
             assert bool((over <= 0).all()), (name, int((over > 0).sum()), float(over.max()))
         assert torch.equal(yf[N:], y0[N:]) and torch.equal(dxf[N:], dx0[N:])
+
+
+@pytest.mark.parametrize("dtype,K,M", [(torch.float32, 44, 20), (torch.float32, 3076, 1028), (torch.bfloat16, 48, 16),
+                                       (torch.bfloat16, 3088, 1040)])
+def test_non_finite_factor_row_stays_in_its_rank(dtype, K, M):
+    """A NaN or infinity in one rank's row of A reaches that column of u only,
+    and one in B that row of dA only, where the last 64 bytes of a row are cut
+    short by the next row's first values."""
+    torch.manual_seed(K)
+    N, r, bad = 70, 20, 7
+    x, dy = torch.randn(N, K, device="cuda").to(dtype), torch.randn(N, M, device="cuda").to(dtype)
+    a, b = torch.randn(r, K, device="cuda").to(dtype), torch.randn(M, r, device="cuda").to(dtype)
+    y = torch.zeros(N, M, device="cuda", dtype=dtype)
+    u = lora_fwd(x, a, b, y.clone(), 0.5)
+    da, db = lora_bwd(x, a, b, u, dy, 0.5)
+    others = [j for j in range(r) if j != bad]
+    for value in (float("nan"), float("inf")):
+        a2, b2 = a.clone(), b.clone()
+        a2[bad, 0], b2[0, bad] = value, value
+        u2 = lora_fwd(x, a2, b, y.clone(), 0.5)
+        da2, db2 = lora_bwd(x, a, b2, u, dy, 0.5)
+        assert torch.equal(u2[:, others], u[:, others]) and not bool(torch.isfinite(u2[:, bad]).any())
+        assert torch.equal(da2[others], da[others]) and not bool(torch.isfinite(da2[bad]).any())
+        assert torch.equal(db2, db)
