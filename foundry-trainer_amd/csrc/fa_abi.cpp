@@ -8,7 +8,9 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "../../include/foundry_attn.h"
 #include "../../include/foundry_block.h"
@@ -229,6 +231,54 @@ size_t bwd_workspace(int32_t dtype, int32_t B, int32_t S, int32_t H, int32_t D) 
     return dtype == FA_DTYPE_F32 ? bwd_min_workspace(dtype, B, S, H, D) : bwd_ds_workspace(dtype, B, S, H, D);
 }
 
+// A launch of 2^32 threads or more wraps without an error, and runs only what
+// is left of its grid.  The attention kernels' launches are below that for
+// B * H * ceil(S / 32) under 2^22 (at most 1024 threads per 32 rows of a head:
+// the f32 pre-pass at D = 128); larger calls run as several, each over some
+// batch items or some heads of one, with the rows, in this order, of its own.
+constexpr int64_t kSliceTiles = (1 << 22) - 1;
+
+template <typename P>
+void move_slice(P &p, size_t elt, int b0, int h0) {
+    const int64_t rows = ((int64_t)b0 * p.H + h0) * p.S;
+    auto at = [&](auto &ptr, int64_t sb, int64_t sh) {
+        using C = std::conditional_t<std::is_same_v<decltype(ptr), void *&>, char *, const char *>;
+        ptr = static_cast<C>(ptr) + (b0 * sb + h0 * sh) * (int64_t)elt;
+    };
+    at(p.q, p.q_sb, p.q_sh);
+    at(p.k, p.k_sb, p.k_sh);
+    at(p.v, p.v_sb, p.v_sh);
+    at(p.o, p.o_sb, p.o_sh);
+    p.lse += rows;
+    if (p.keep) p.keep += (int64_t)b0 * p.S;
+    if constexpr (std::is_same_v<P, fa::AttnBwdParams>) {
+        at(p.dout, p.do_sb, p.do_sh);
+        at(p.dq, p.dq_sb, p.dq_sh);
+        at(p.dk, p.dk_sb, p.dk_sh);
+        at(p.dv, p.dv_sb, p.dv_sh);
+        p.delta += rows;
+        p.lse2 += rows;
+        p.ds = nullptr;  // dQ recomputes: the same bits
+    }
+}
+
+template <typename P, typename F>
+hipError_t launch_in_slices(const P &p, int32_t dtype, F launch) {
+    const int64_t most = std::max<int64_t>(kSliceTiles / ((p.S + 31) / 32), 1);  // heads per launch, over all batch items
+    if ((int64_t)p.B * p.H <= most) return launch(p);
+    const int nh = (int)std::min<int64_t>(p.H, most), nb = (int)std::max<int64_t>(most / p.H, 1);
+    for (int64_t b0 = 0; b0 < p.B; b0 += nb)
+        for (int64_t h0 = 0; h0 < p.H; h0 += nh) {
+            P part = p;
+            move_slice(part, dtype == FA_DTYPE_BF16 ? 2 : 4, (int)b0, (int)h0);
+            part.B = (int)std::min<int64_t>(nb, p.B - b0);
+            part.H = (int)std::min<int64_t>(nh, p.H - h0);
+            const hipError_t e = launch(part);
+            if (e != hipSuccess) return e;
+        }
+    return hipSuccess;
+}
+
 // forward workspace of a split call: O partials [split][B,H,S][D] f32, then
 // the partial LSEs [split][B,H,S] f32; 0 when the call does not split
 size_t fwd_workspace(int32_t dtype, int32_t B, int32_t S, int32_t H, int32_t D) {
@@ -313,8 +363,10 @@ fa_status fa_attn_fwd(const fa_attn_fwd_args *a, void *stream) {
         }
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const hipError_t e = a->dtype == FA_DTYPE_BF16 ? fa::launch_attn_fwd_bf16(p, a->head_dim, s)
-                                                   : fa::launch_attn_fwd_f32(p, a->head_dim, s);
+    const hipError_t e = launch_in_slices(p, a->dtype, [&](const fa::AttnFwdParams &part) {
+        return a->dtype == FA_DTYPE_BF16 ? fa::launch_attn_fwd_bf16(part, a->head_dim, s)
+                                         : fa::launch_attn_fwd_f32(part, a->head_dim, s);
+    });
     if (e != hipSuccess) return hip_fail(e, "attention forward launch");
     return ok();
 }
@@ -424,8 +476,10 @@ fa_status fa_attn_bwd_phase(const fa_attn_bwd_args *a, int32_t phase, void *stre
     fill_bwd_params(a, static_cast<char *>(a->workspace), split_for(a->dtype, a->batch, a->seq, a->heads),
                     ds > 0 && a->workspace_bytes >= need + ds, p);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const hipError_t e = a->dtype != FA_DTYPE_BF16 ? fa::launch_attn_bwd_f32(p, a->head_dim, phase, s)
-                                                   : fa::launch_attn_bwd_bf16(p, a->head_dim, phase, s);
+    const hipError_t e = launch_in_slices(p, a->dtype, [&](const fa::AttnBwdParams &part) {
+        return a->dtype != FA_DTYPE_BF16 ? fa::launch_attn_bwd_f32(part, a->head_dim, phase, s)
+                                         : fa::launch_attn_bwd_bf16(part, a->head_dim, phase, s);
+    });
     if (e != hipSuccess) return hip_fail(e, "attention backward launch");
     return ok();
 }
