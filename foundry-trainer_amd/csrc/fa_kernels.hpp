@@ -78,6 +78,10 @@ hipError_t launch_attn_bwd_f32(const AttnBwdParams &p, int D, int phase, hipStre
 // the f32 backward's phase 1 (attn_bwd.hip)
 hipError_t launch_attn_bwd_delta_f32(const AttnBwdParams &p, int D, hipStream_t s);
 
+// Most threads of a launch along one dimension: past it the grid wraps, without
+// an error, and only what is left of it runs.
+constexpr int64_t kMaxThreads = (int64_t(1) << 32) - 1;
+
 // CU count of the current device (cached per device; 256 if unknown).
 int device_cu_count();
 

@@ -32,6 +32,7 @@
 //           grid.
 // The general f32 kernels (lora_rowdot_kernel, lora_expand_kernel,
 // lora_colsum_kernel) serve widths and strides the others do not address.
+#include <algorithm>
 #include <type_traits>
 
 #include "fa_device.hpp"
@@ -1257,7 +1258,8 @@ hipError_t launch_lora_grad_many_bf16(const LoraGradItem *items, int count, void
         GradMany g{};
         g.count = count - k0 < kGradMany ? count - k0 : kGradMany;
         char *ws = static_cast<char *>(work);
-        int wgs = 0, max_out = 1, max_npad = kCsRows;
+        int wgs = 0, max_npad = kCsRows;
+        int64_t max_out = 1;
         bool staged = false;
         for (int k = 0; k < g.count; ++k) {
             const LoraGradItem &it = items[k0 + k];
@@ -1286,9 +1288,10 @@ hipError_t launch_lora_grad_many_bf16(const LoraGradItem *items, int count, void
             q.part = reinterpret_cast<float *>(ws);
             ws += al256((size_t)q.splits * it.C * q.rw * 4);
             wgs += (it.C + kCsCols - 1) / kCsCols * q.splits;
-            max_out = it.C * q.rw > max_out ? it.C * q.rw : max_out;
+            max_out = std::max(max_out, (int64_t)it.C * q.rw);
             max_npad = q.npad > max_npad ? q.npad : max_npad;
         }
+        if (max_out > kMaxThreads - 255) return hipErrorInvalidConfiguration;  // the reduce's grid
         if (staged)
             hipLaunchKernelGGL(lora_ut_many_kernel, dim3((unsigned)((64 * max_npad + 255) / 256), (unsigned)g.count),
                                dim3(256), 0, st, g);

@@ -3,7 +3,7 @@ which a grid wraps without an error and runs only what is left of it."""
 import pytest
 import torch
 
-from foundry_attn import attn_bwd, attn_fwd
+from foundry_attn import attn_bwd, attn_fwd, lora_bwd
 
 pytestmark = pytest.mark.gpu
 
@@ -36,3 +36,15 @@ def test_attention_over_many_heads(dtype, B, H, masked):
     # dS is the rounding of two 64-term sums of dO V (|dO V| sums below 200), dQ and dK 0.125 dS |x| (below 6.5)
     for g in (dq, dk):
         assert float(g.abs().max()) <= 0.125 * 6.5 * 128 * 200 * 2.0 ** -24
+
+
+def test_lora_gradient_of_2_26_features():
+    """dA of one token and rank 1 is that token: C x 32 partial sums, 2^31."""
+    K = 1 << 26
+    x = torch.randn(1, K, device="cuda", dtype=torch.bfloat16)
+    a = torch.zeros(1, K, device="cuda", dtype=torch.bfloat16)
+    b, dy = (torch.zeros(*s, device="cuda", dtype=torch.bfloat16) for s in ((16, 1), (1, 16)))
+    b[3, 0] = dy[0, 3] = 1
+    da, db = lora_bwd(x, a, b, torch.full((1, 1), 2.0, device="cuda"), dy, 1.0)
+    assert torch.equal(da, x.float())
+    assert torch.equal(db, 2 * dy.float().t())
