@@ -973,9 +973,10 @@ hipError_t rowdot16(const T *X, int64_t ldx, const T *W, TO *out, int64_t ldo, i
 
 hipError_t rowdot(const float *X, int64_t ldx, const float *W, float *out, int64_t ldo, int N, int K, int R, float s,
                   hipStream_t st) {
-    // 16-byte W rows, and 64 rows of X and all of W within 32-bit byte offsets
+    // 16-byte W rows, 64 rows of X and all of W within 32-bit byte offsets, and
+    // 512 threads per 64 rows (the form so many rows take) within a launch
     const int64_t xspan = (int64_t)63 * ldx + K, wspan = (int64_t)R * K;
-    if (K % 4 == 0 && xspan < (1 << 30) && wspan < (1 << 30))
+    if (K % 4 == 0 && xspan < (1 << 30) && wspan < (1 << 30) && (int64_t)N * 8 <= kMaxThreads - 511)
         return rowdot16<float, float>(X, ldx, W, out, ldo, N, K, R, s, st);
     hipLaunchKernelGGL(lora_rowdot_kernel, dim3((N + 127) / 128), dim3(256), 0, st, X, ldx, W, out, ldo, N, K, R, s);
     return hipGetLastError();

@@ -48,3 +48,17 @@ def test_lora_gradient_of_2_26_features():
     da, db = lora_bwd(x, a, b, torch.full((1, 1), 2.0, device="cuda"), dy, 1.0)
     assert torch.equal(da, x.float())
     assert torch.equal(db, 2 * dy.float().t())
+
+
+def test_lora_f32_gradient_of_2_29_tokens():
+    """du of the last tokens, which a wrapped grid of the down product would
+    leave out, reaches dA: all other tokens are zero."""
+    N, K, M = (1 << 29) + 5, 4, 4
+    x, dy = torch.zeros(N, K, device="cuda"), torch.zeros(N, M, device="cuda")
+    u = torch.zeros(N, 1, device="cuda")
+    x[-3:, 1] = torch.tensor([1.0, 2.0, 3.0], device="cuda")
+    dy[-3:, 0] = 1
+    u[-3:] = 1
+    a, b = torch.ones(1, K, device="cuda"), torch.tensor([[2.0], [1.0], [1.0], [1.0]], device="cuda")
+    da, db = lora_bwd(x, a, b, u, dy, 1.0)
+    assert da.tolist() == [[0.0, 12.0, 0.0, 0.0]] and db.tolist() == [[3.0], [0.0], [0.0], [0.0]]
