@@ -302,11 +302,20 @@ def _codes(t) -> str:
 
 def packer(cls):
     """pack(values in field order, nested ones flattened, pointers as ints) ->
-    bytes laid out as the structure cls."""
+    bytes laid out as the structure cls.  A value that its field does not hold
+    (2^31 rows) is FA_ERR_INVALID_ARG."""
     st = struct.Struct("@" + _codes(cls) + "0q")
     if st.size != ctypes.sizeof(cls):
         raise AssertionError(f"{cls.__name__}: packed size {st.size}, structure {ctypes.sizeof(cls)}")
-    return st.pack
+    pack = st.pack
+
+    def packed(*values):
+        try:
+            return pack(*values)
+        except struct.error as e:
+            raise FoundryAttnError(FA_ERR_INVALID_ARG, f"{cls.__name__}: {e}") from None
+
+    return packed
 
 
 @functools.lru_cache(maxsize=None)

@@ -160,3 +160,14 @@ def test_ln_mod_bwd_gate_rejects(case):
         dy = torch.zeros(128, 64, dtype=bf).t()
     with pytest.raises(FoundryAttnError):
         fb.ln_mod_bwd_gate(x, dy, sc, mean, rstd, g, 1e-6, **kw)
+
+
+@pytest.mark.parametrize("op", ["gelu", "silu", "swiglu", "ln_mod_fwd"])
+def test_rows_past_32_bits_are_refused(op):
+    """2^31 rows (one row of memory, repeated) do not fit the library's 32-bit
+    counts: refused like any other bad argument."""
+    from foundry_attn import block as fb
+    x, v = torch.zeros(1, 8, dtype=bf).expand(1 << 31, 8), torch.zeros(8, dtype=bf)
+    args = {"swiglu": (x, x), "ln_mod_fwd": (x, v, v)}.get(op, (x,))
+    with pytest.raises(FoundryAttnError):
+        getattr(fb, op)(*args, out=x)
