@@ -90,3 +90,25 @@ def test_non_finite_factor_row_stays_in_its_rank(dtype, K, M):
         assert torch.equal(u2[:, others], u[:, others]) and not bool(torch.isfinite(u2[:, bad]).any())
         assert torch.equal(da2[others], da[others]) and not bool(torch.isfinite(da2[bad]).any())
         assert torch.equal(db2, db)
+
+
+@pytest.mark.parametrize("stride", [1 << 24, 1 << 26])
+def test_lora_f32_row_strides_past_32_bit_offsets(stride):
+    """Rows of x, dy, y and dx far apart: 64 of them past 4 GiB (the general
+    down and up products), and 16 (the general gradient as well)."""
+    N, K, M, r = 3, 8, 12, 5
+    torch.manual_seed(stride >> 20)
+    buf = torch.empty((N - 1) * stride + 128, device="cuda")
+    x, dy, y, dx = (buf.as_strided((N, w), (stride, 1), at) for w, at in ((K, 0), (M, 16), (M, 32), (K, 48)))
+    for t in (x, dy, y, dx):
+        t.copy_(torch.randn(t.shape, device="cuda"))
+    a, b = torch.randn(r, K, device="cuda"), torch.randn(M, r, device="cuda")
+    X, DY, Y, DX, A, B = (t.double().cpu() for t in (x, dy, y, dx, a, b))
+    u = lora_fwd(x, a, b, y, 0.5)
+    da, db = lora_bwd(x, a, b, u, dy, 0.5, dx=dx)
+    U, DU = X @ A.t(), 0.5 * (DY @ B)
+    for name, got, want in (("u", u, U), ("y", y, Y + 0.5 * U @ B.t()), ("da", da, DU.t() @ X),
+                            ("db", db, 0.5 * DY.t() @ U), ("dx", dx, DX + DU @ A)):
+        err = float((got.double().cpu() - want).norm() / want.norm())
+        assert err <= (max(N, K, M) + r) * 2.0 ** -24, (name, err)
+    assert torch.equal(x.double().cpu(), X) and torch.equal(dy.double().cpu(), DY)
