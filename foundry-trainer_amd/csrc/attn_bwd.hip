@@ -986,7 +986,7 @@ hipError_t launch_attn_bwd_bf16(const AttnBwdParams &p, int D, int phase, hipStr
     // the pre-pass for its own queries, then dK/dV; with 4-wave kernels the
     // pre-pass, then dK/dV and dQ in one grid.  (Against dQ on a second stream
     // beside dK/dV, joined by events, the one grid saves 45 us of host time a
-    // call, and on the GPU B2 H24 S333 49 -> 32 us, B4 H24 S1536 409 -> 406.)
+    // call, and on the GPU B2 H24 S333 49 -> 32 us; B4 H24 S1536 is unchanged.)
     const bool fused = phase == 0 && nw == 8, pair = phase == 0 && nw == 4;
     hipError_t e = hipSuccess;
     if (pair || phase == 1) {

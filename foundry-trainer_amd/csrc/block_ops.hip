@@ -196,8 +196,8 @@ __device__ __forceinline__ void raw_keep(RawF32 &r) { asm volatile("" : "+v"(r.w
 // HBM-bound.  All of a row's operands, the residual's gradient among them, are
 // loaded before any is used and stay in storage form (x and dy are widened
 // again after the sums): five waves per SIMD hold a 4608-row grid in one
-// round.  4608 x 3072 bf16 from cold HBM 31.1 -> 27.2 us (5.3 TB/s), with
-// GATE_OUT 38.9 -> 32.0, against loads chunk by chunk as the sums need them.
+// round.  4608 x 3072 bf16 from cold HBM 31.1 -> 27.2 us (4.2 TB/s), with
+// GATE_OUT 38.9 -> 32.0 (4.4), against loads chunk by chunk as the sums need them.
 // A row spread over six waves took 25.2 and 30.0, but adds in another order:
 // dx then differs in bf16 roundings.
 //
@@ -346,7 +346,7 @@ __global__ __launch_bounds__(kEltLanes) void elementwise_kernel(EltParams p) {
 // divided a 64-bit index by the row length on each), and what the backward
 // reads last and both write goes past the caches: 4608 x 9216 bf16 from cold
 // HBM 54 -> 50 -> 44 us forward (5.8 TB/s), 81 -> 74 -> 63 us backward (6.7 TB/s),
-// and the layer-norm backward after it 27 -> 21.
+// and the layer-norm backward after it 27 -> 22.
 template <typename T, bool BWD>
 __global__ __launch_bounds__(kEltLanes) void swiglu_kernel(SwigluParams p) {
     const int e = (blockIdx.x * kEltLanes + threadIdx.x) * 8;

@@ -130,7 +130,7 @@ typedef struct fa_attn_bwd_args {
     const uint8_t *key_keep;                    /* the forward's mask or NULL    */
     void *dq, *dk, *dv;                         /* [B,S,H,D] outputs             */
     void *workspace;                            /* device scratch, 256-B aligned */
-    size_t workspace_bytes;                     /* >= fa_attn_bwd_workspace_size */
+    size_t workspace_bytes;                     /* >= fa_attn_bwd_min_workspace_size */
     fa_strides q_stride, k_stride, v_stride, o_stride, do_stride;
     fa_strides dq_stride, dk_stride, dv_stride;
 } fa_attn_bwd_args;
