@@ -166,8 +166,8 @@ __global__ __launch_bounds__(256) void ln_mod_fwd_kernel(LnModParams p) {
     }
 }
 
-// 8 consecutive elements as they lie in memory, at byte offset off of a row's
-// buffer descriptor: past its end they read as zero.
+// Elements e .. e + 7 of a row as they lie in memory, through its buffer
+// descriptor: past the row's end they read as zero.
 struct RawBf16 {
     u32x4 w;
 };
@@ -195,11 +195,12 @@ __device__ __forceinline__ void raw_keep(RawF32 &r) { asm volatile("" : "+v"(r.w
 //
 // HBM-bound.  All of a row's operands, the residual's gradient among them, are
 // loaded before any is used and stay in storage form (x and dy are widened
-// again after the sums): five waves per SIMD hold a 4608-row grid in one
-// round.  4608 x 3072 bf16 from cold HBM 31.1 -> 27.2 us (4.2 TB/s), with
-// GATE_OUT 38.9 -> 32.0 (4.4), against loads chunk by chunk as the sums need them.
-// A row spread over six waves took 25.2 and 30.0, but adds in another order:
-// dx then differs in bf16 roundings.
+// again after the sums): 91 VGPRs for a bf16 row of 3072, so five waves per
+// SIMD hold a 4608-row grid in one round (101 and four with GATE_OUT; held to
+// five it spills and takes 35.2 us).  4608 x 3072 bf16 from cold HBM 31.1 ->
+// 27.2 us (4.2 TB/s), with GATE_OUT 38.9 -> 32.0 (4.4), against loads chunk by
+// chunk as the sums need them.  A row spread over six waves took 25.2 and
+// 30.0, but adds in another order: dx then differs in bf16 roundings.
 //
 // GATE_OUT: also gdx = g * dx, from dx as rounded to T (the same fma as the
 // gated-residual op with no x), the gradient through a gated branch whose
